@@ -147,6 +147,12 @@ void set_kernel_attrs() {
     if (g_attr_err == hipSuccess)
       g_attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd::prefixlm_bwd_dq_ds_kernel<64>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, bwd::q2::Geo<64>::LDS_BYTES);
+    if (g_attr_err == hipSuccess)
+      g_attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&kvc::extend_kernel<1>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, kvc::ExtGeo<1>::LDS_BYTES);
+    if (g_attr_err == hipSuccess)
+      g_attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&kvc::extend_kernel<2>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, kvc::ExtGeo<2>::LDS_BYTES);
   });
 }
 
@@ -912,10 +918,38 @@ int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
   return PREFIXLM_OK;
 }
 
+// Whether the 256-byte rows of a [B, N, H] cache with these element strides are all apart:
+// with the dimensions ordered by stride, each stride covers the extent of the smaller ones.
+static bool rows_apart(int64_t B, int64_t N, int64_t H, int64_t sb, int64_t sn, int64_t sh) {
+  std::pair<int64_t, int64_t> d[3] = {{sb, B}, {sn, N}, {sh, H}};   // (stride, count)
+  std::sort(d, d + 3);
+  int64_t extent = kvc::D;
+  for (const auto& x : d) {
+    if (x.second == 1) continue;
+    if (x.first < extent) return false;
+    extent += x.first * (x.second - 1);
+  }
+  return true;
+}
+
+// Query waves of the extend kernel for S new rows, its query blocks, and the key splits of
+// either kernel.
+static int ext_qw(int S) { return S <= 32 ? 1 : S <= 64 ? 2 : 4; }
+static int kv_nqb(int S) { return S == 1 ? 1 : (S + 32 * ext_qw(S) - 1) / (32 * ext_qw(S)); }
+static int64_t kv_nsplit(int64_t B, int S, int64_t H, int64_t Smax) {
+  if (S == 1) return (Smax + kvc::kChunk - 1) / kvc::kChunk;
+  const int64_t tk = 32 * (4 / ext_qw(S)), units = B * H * kv_nqb(S);
+  // 512 workgroups fill the chip (two per CU); more splits only add partials to write and
+  // merge: 4 x 16 heads x 45 queries 38 us a call at 512, 42 at 1024, 60 at 2048, and 2 x 16 x
+  // 300 on 8192 rows 97 us at 512 against 103 at 256
+  const int64_t want = (512 + units - 1) / units, most = (Smax + tk - 1) / tk;
+  return std::max<int64_t>(1, std::min({want, most, (int64_t)kvc::kMaxSplits}));
+}
+
 size_t prefixlm_kvcache_workspace_size(int32_t batch, int32_t seqlen_q, int32_t num_heads, int32_t head_dim,
                                        int32_t max_seqlen_cache) {
   if (batch < 1 || seqlen_q < 1 || num_heads < 1 || max_seqlen_cache < 1) return 0;
-  const int64_t nsplit = (max_seqlen_cache + kvc::kChunk - 1) / kvc::kChunk;
+  const int64_t nsplit = kv_nsplit(batch, seqlen_q, num_heads, max_seqlen_cache);
   const size_t decode = align_up(sizeof(float) * (size_t)batch * seqlen_q * num_heads * nsplit * kvc::kPart);
   const int64_t T = (int64_t)batch * seqlen_q;
   size_t prefill = 0;
@@ -972,26 +1006,36 @@ int prefixlm_kvcache_fwd(const prefixlm_kvcache_args* a, void* stream_) {
   P.vc_sb = a->v_cache_stride_b; P.vc_ss = a->v_cache_stride_s; P.vc_sh = a->v_cache_stride_h;
   P.o_sb = a->out_stride_b; P.o_ss = a->out_stride_s; P.o_sh = a->out_stride_h;
   P.B = B; P.S = S; P.H = H; P.Smax = Smax;
-  P.nsplit = (Smax + kvc::kChunk - 1) / kvc::kChunk;
+  P.nsplit = (int)kv_nsplit(B, S, H, Smax);
+  P.nqb = kv_nqb(S);
   P.causal = a->is_causal ? 1 : 0;
   P.seqlen_const = a->cache_seqlen;
   P.s_new = has_new ? S : 0;
   P.scale_log2 = a->softmax_scale * kLog2e;
 
   (void)hipGetLastError();
-  if (has_new) {
-    const int64_t threads = (int64_t)B * S * H * 16;
-    if ((threads + 255) / 256 > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "too many rows");
-    hipLaunchKernelGGL(kvc::append_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, P);
-  }
   // the reference's prefill: an empty cache and a packed batch of new rows
   const bool packed = B == 1 || (a->q_stride_b == (int64_t)S * a->q_stride_s &&
                                  a->k_stride_b == (int64_t)S * a->k_stride_s &&
                                  a->v_stride_b == (int64_t)S * a->v_stride_s &&
                                  a->out_stride_b == (int64_t)S * a->out_stride_s);
   const int64_t T = (int64_t)B * S;
-  if (!a->cache_seqlens && a->cache_seqlen == 0 && has_new && packed && S <= Smax && T < 0x7fffffff &&
-      a->q_stride_s >= kvc::D && a->k_stride_s >= kvc::D && a->v_stride_s >= kvc::D && a->out_stride_s >= kvc::D) {
+  const bool prefill = !a->cache_seqlens && a->cache_seqlen == 0 && has_new && packed && S <= Smax &&
+                       T < 0x7fffffff && a->q_stride_s >= kvc::D && a->k_stride_s >= kvc::D &&
+                       a->v_stride_s >= kvc::D && a->out_stride_s >= kvc::D;
+  // The extend kernel reads the new rows from k, v and writes them to the caches in one
+  // launch; that needs cache rows of its own for every (b, row, head) and two caches (a
+  // row shared between batch rows would be read by one while the other writes it).
+  P.fused = !prefill && S > 1 && has_new &&
+            rows_apart(B, Smax, H, a->k_cache_stride_b, a->k_cache_stride_s, a->k_cache_stride_h) &&
+            rows_apart(B, Smax, H, a->v_cache_stride_b, a->v_cache_stride_s, a->v_cache_stride_h) &&
+            a->k_cache != a->v_cache;
+  if (has_new && !P.fused) {
+    const int64_t threads = (int64_t)B * S * H * 16;
+    if ((threads + 255) / 256 > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "too many rows");
+    hipLaunchKernelGGL(kvc::append_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, P);
+  }
+  if (prefill) {
     char* ws = static_cast<char*>(a->workspace);
     int32_t* meta = reinterpret_cast<int32_t*>(ws);
     size_t off = align_up(sizeof(int32_t) * 3 * (size_t)(B + 1));
@@ -1022,11 +1066,23 @@ int prefixlm_kvcache_fwd(const prefixlm_kvcache_args* a, void* stream_) {
     return prefixlm_fwd(&f, stream_);
   }
   {
-    const int64_t nblk = (int64_t)B * H * P.nsplit;
+    const int64_t units = (int64_t)B * H * P.nsplit, nblk = S == 1 ? units : (units + 7) / 8 * 8 * P.nqb;
     if (nblk > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "grid too large");
-    hipLaunchKernelGGL(kvc::decode_kernel, dim3((unsigned)nblk), dim3(kvc::NT), 0, stream, P);
-    const int64_t waves = (int64_t)B * S * H;
-    hipLaunchKernelGGL(kvc::combine_kernel, dim3((unsigned)((waves * 64 + 255) / 256)), dim3(256), 0, stream, P);
+    set_kernel_attrs();
+    if (g_attr_err != hipSuccess)
+      return fail(PREFIXLM_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(g_attr_err));
+    if (S == 1)
+      hipLaunchKernelGGL(kvc::decode_kernel, dim3((unsigned)nblk), dim3(kvc::NT), 0, stream, P);
+    else if (ext_qw(S) == 1)
+      hipLaunchKernelGGL(kvc::extend_kernel<1>, dim3((unsigned)nblk), dim3(kvc::NT), kvc::ExtGeo<1>::LDS_BYTES, stream, P);
+    else if (ext_qw(S) == 2)
+      hipLaunchKernelGGL(kvc::extend_kernel<2>, dim3((unsigned)nblk), dim3(kvc::NT), kvc::ExtGeo<2>::LDS_BYTES, stream, P);
+    else
+      hipLaunchKernelGGL(kvc::extend_kernel<4>, dim3((unsigned)nblk), dim3(kvc::NT), kvc::ExtGeo<4>::LDS_BYTES, stream, P);
+    if (S == 1 || P.nsplit > 1) {
+      const int64_t waves = (int64_t)B * S * H;
+      hipLaunchKernelGGL(kvc::combine_kernel, dim3((unsigned)((waves * 64 + 255) / 256)), dim3(256), 0, stream, P);
+    }
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(PREFIXLM_ERR_HIP, "kv-cache launch: %s", hipGetErrorString(e));

@@ -1,0 +1,109 @@
+"""GPU: several new rows per sequence onto filled caches (the extend kernel) against the
+oracle, at the edges of its query blocks (32, 64, 128 rows), key tiles (32, 64, 128 keys)
+and key splits, with rows that fall past the cache, cached-only calls, strided and shared
+caches, and non-finite values.
+
+Tolerance per element: half a bf16 ulp of the reference (2^-8 |ref|, the output's own
+rounding) plus 2^-14 max|V|: P enters P V as two bf16 terms, which leaves at most 2^-17 of
+each probability, and fp32 sums of up to 1500 terms in another order stay below 2^-15."""
+import pytest
+import torch
+
+from oracle.kvcache_oracle import kvcache_attention
+from prefixlm import flash_attn_with_kvcache
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _inputs(B, S, H, Smax, seed):
+    g = torch.Generator().manual_seed(seed)
+    mk = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)  # noqa: E731
+    return mk(B, S, H, 128), mk(B, S, H, 128), mk(B, S, H, 128), mk(B, Smax, H, 128), mk(B, Smax, H, 128)
+
+
+def _check(got, ref, v_max):
+    got = got.float().cpu()
+    err, tol = (got - ref).abs(), ref.abs() * 2.0 ** -8 + v_max * 2.0 ** -14
+    assert (err <= tol).all(), f"worst {(err - tol).max().item():.3e} over, max_abs {err.max().item():.3e}"
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("S", [2, 31, 32, 33, 64, 65, 127, 128, 130])
+def test_extend_matches_oracle(S, causal):
+    B, H, Smax = 4, 3, 700
+    q, k, v, kc, vc = _inputs(B, S, H, Smax, S)
+    lens = torch.tensor([0, 127, 500, Smax - S], dtype=torch.int32)
+    ref, kr, vr = kvcache_attention(q, kc, vc, k, v, lens, causal)
+    d = [t.to(DEV) for t in (q, k, v, kc, vc)]
+    out = flash_attn_with_kvcache(d[0], d[3], d[4], k=d[1], v=d[2], cache_seqlens=lens.to(DEV), causal=causal)
+    assert torch.equal(d[3].cpu(), kr) and torch.equal(d[4].cpu(), vr)
+    _check(out, ref, v.abs().max().item())
+
+
+@pytest.mark.parametrize("B,S,H,Smax", [(2, 40, 16, 1500), (70, 70, 16, 70), (9, 300, 16, 320)])
+def test_extend_splits(B, S, H, Smax):
+    """Many splits of few units, and more units than the grid wants (one split, written directly)."""
+    q, k, v, kc, vc = _inputs(B, S, H, Smax, B)
+    lens = torch.arange(B, dtype=torch.int32) * 7 % (Smax - S + 1)
+    ref, kr, vr = kvcache_attention(q, kc, vc, k, v, lens, True)
+    d = [t.to(DEV) for t in (q, k, v, kc, vc)]
+    out = flash_attn_with_kvcache(d[0], d[3], d[4], k=d[1], v=d[2], cache_seqlens=lens.to(DEV), causal=True)
+    assert torch.equal(d[3].cpu(), kr) and torch.equal(d[4].cpu(), vr)
+    _check(out, ref, v.abs().max().item())
+
+
+@pytest.mark.parametrize("new", [True, False])
+def test_extend_past_the_cache_and_cached_only(new):
+    """Rows past Smax are dropped; without new rows the queries see the cached ones."""
+    B, S, H, Smax = 3, 20, 2, 200
+    q, k, v, kc, vc = _inputs(B, S, H, Smax, 3)
+    lens = torch.tensor([190, 60, 200], dtype=torch.int32)
+    ref, kr, vr = kvcache_attention(q, kc, vc, k if new else None, v if new else None, lens, False)
+    d = [t.to(DEV) for t in (q, k, v, kc, vc)]
+    out = flash_attn_with_kvcache(d[0], d[3], d[4], k=d[1] if new else None, v=d[2] if new else None,
+                                  cache_seqlens=lens.to(DEV))
+    assert torch.equal(d[3].cpu(), kr) and torch.equal(d[4].cpu(), vr)
+    _check(out, ref, 5.0)
+
+
+@pytest.mark.parametrize("layout", ["heads_first", "shared_batch", "negative_scale"])
+def test_extend_strides(layout):
+    """Caches laid out [B, H, Smax, D]; one cache row shared by the whole batch (appended
+    before it is read, so every sequence must see the same rows); a negative softmax scale."""
+    B, S, H, Smax = 2, 33, 3, 300
+    q, k, v, kc, vc = _inputs(B, S, H, Smax, 11)
+    lens = torch.tensor([100, 230], dtype=torch.int32)
+    scale = -0.05 if layout == "negative_scale" else None
+    if layout == "shared_batch":
+        k, v, lens = k[:1].expand(B, -1, -1, -1), v[:1].expand(B, -1, -1, -1), torch.tensor([100, 100], dtype=torch.int32)
+        kc, vc = kc[:1].expand(B, -1, -1, -1), vc[:1].expand(B, -1, -1, -1)
+        kd, vd = (x[:1].to(DEV).expand(B, -1, -1, -1) for x in (kc, vc))
+    elif layout == "heads_first":
+        kd, vd = (x.to(DEV).transpose(1, 2).contiguous().transpose(1, 2) for x in (kc, vc))
+    else:
+        kd, vd = kc.to(DEV), vc.to(DEV)
+    ref, kr, vr = kvcache_attention(q, kc, vc, k, v, lens, True, scale)
+    out = flash_attn_with_kvcache(q.to(DEV), kd, vd, k=k.to(DEV), v=v.to(DEV), cache_seqlens=lens.to(DEV), causal=True,
+                                  softmax_scale=scale)
+    assert torch.equal(kd.cpu(), kr) and torch.equal(vd.cpu(), vr)
+    _check(out, ref, v.abs().max().item())
+
+
+@pytest.mark.parametrize("S", [6, 50, 100])
+def test_extend_non_finite_values(S):
+    """A value row that is infinite reaches the queries that see it, as +-inf and not as NaN,
+    and no other query."""
+    B, H, Smax = 2, 2, 400
+    q, k, v, kc, vc = _inputs(B, S, H, Smax, 21)
+    lens = torch.tensor([150, 301], dtype=torch.int32)
+    bad = S - 3                                    # the new row only the last three queries see
+    v[:, bad] = float("inf")
+    v[:, bad, :, 5] = float("-inf")
+    ref, _, _ = kvcache_attention(q, kc, vc, k, v.nan_to_num(posinf=0.0, neginf=0.0), lens, True)
+    d = [t.to(DEV) for t in (q, k, v, kc, vc)]
+    out = flash_attn_with_kvcache(d[0], d[3], d[4], k=d[1], v=d[2], cache_seqlens=lens.to(DEV), causal=True).float().cpu()
+    _check(out[:, :bad], ref[:, :bad], 5.0)
+    want = torch.full_like(out[:, bad:], float("inf"))
+    want[..., 5] = float("-inf")
+    assert torch.equal(out[:, bad:], want)
