@@ -11,11 +11,11 @@
 //
 // Kernels:
 //   append  : copies the new k, v rows into the caches (rows past Smax are dropped);
-//   decode  : one query per row, split-K over the keys. A workgroup = (b, h, split of kChunk
-//             keys); each 16-lane group owns one key at a time (16 x 16-byte chunks of a
-//             256-byte row), four keys per step, with an online softmax in fp32; the 16
-//             groups are merged through LDS and the split writes (max, sum, o[D])
-//             unnormalised to the workspace. HBM-bound: 2 * D * 2 bytes per key.
+//   decode  : one query per row, split-K over the keys. A workgroup = (b, h, split); each
+//             16-lane group owns one key at a time (16 x 16-byte chunks of a 256-byte row),
+//             four keys per step, with an online softmax in fp32; the 16 groups are merged
+//             and the split writes (max, sum, o[D]) unnormalised to the workspace, or out
+//             when it is the only one. HBM-bound: 2 * D * 2 bytes per key.
 //   extend  : several queries per row (S >= 2): the same split-K on the matrix cores, every
 //             staged key serving 32 QW queries (see the kernel);
 //   combine : merges the splits of each (b, i, h) and writes bf16 out.
@@ -29,7 +29,7 @@ constexpr int D = 128;
 constexpr int NT = 256;
 constexpr int GROUPS = NT / 16;      // keys in flight per workgroup step (x kUnroll)
 constexpr int kUnroll = 4;
-constexpr int kChunk = 512;          // keys per split
+constexpr int kStep = GROUPS * kUnroll;   // keys per workgroup step
 constexpr int kPart = D + 4;         // floats per partial: max (log2 units), sum, 2 unused, o[D]
 static_assert(kPart % 4 == 0, "partials keep o 16-byte aligned");
 
@@ -46,7 +46,7 @@ struct Params {
   int64_t kc_sb, kc_ss, kc_sh, vc_sb, vc_ss, vc_sh, o_sb, o_ss, o_sh;
   int B, S, H, Smax, nsplit, causal, seqlen_const;
   int s_new;              // rows appended by this call: S, or 0 without new k, v
-  int fused;              // extend: new rows are read from k, v and written to the caches by the same kernel
+  int fused;              // new rows are read from k, v and written to the caches by the same kernel
   int nqb;                // extend: query blocks of 32 QW rows
   float scale_log2;
 };
@@ -72,27 +72,43 @@ __global__ __launch_bounds__(256) void append_kernel(Params P) {
   *reinterpret_cast<u32x4*>(P.vc + b * P.vc_sb + row * P.vc_ss + h * P.vc_sh + 8 * c) = vv;
 }
 
-__device__ __forceinline__ float sum16(float x) {
-#pragma unroll
-  for (int m = 1; m < 16; m <<= 1) x += __shfl_xor(x, m);
-  return x;
+// 16 bytes of a cached row: read once per call, by one workgroup
+__device__ __forceinline__ u32x4 load_once(const bf16* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
 }
 
-// blockIdx.x = ((b * H + h) * nsplit + split); one query per row (S = 1)
+// One query per row (S = 1): blockIdx.x = ((b * H + h) * nsplit + split). The splits share
+// each sequence's own length evenly (in steps of 64 keys), so a ragged batch has no
+// workgroups without keys beside full ones. Bound by HBM. The cache loads are non-temporal:
+// a row is read once, and kept out of the caches it costs no write-back of what it would
+// evict. 64 x 16 heads, 2100-4000 of 4096 rows (1.6 GB): 262 us with the combine, 6.1 TB/s,
+// against 285 with plain loads and 322 for fixed 512-key splits, plain loads and an append
+// launch. Loading the next 64 keys at the end of a step instead of at its start is worth 2%;
+// doing it before the step's P V, or the heads as the fastest grid index, changes nothing.
 __global__ __launch_bounds__(NT) void decode_kernel(Params P) {
-  __shared__ float s_m[GROUPS], s_l[GROUPS];
-  __shared__ f32x4 s_o[GROUPS][D / 4];
+  __shared__ float s_m[NT / 64], s_l[NT / 64];
+  __shared__ f32x4 s_o[NT / 64][D / 4];
   const int split = blockIdx.x % P.nsplit;
   const int bh = blockIdx.x / P.nsplit;
   const int h = bh % P.H, b = bh / P.H;
   const int tid = threadIdx.x, grp = tid >> 4, g16 = tid & 15;
   const int len = cache_len(P, b);
-  const int lk = min(P.Smax, len + P.s_new);   // keys in the cache after the append
+  // keys read from the cache; with P.fused the new row is not one of them
+  const int lk = min(P.Smax, len + (P.fused ? 0 : P.s_new));
+  const int per = ((lk + P.nsplit - 1) / P.nsplit + kStep - 1) / kStep * kStep;
+  const int k0 = split * per, k1 = min(lk, k0 + per);
   const bf16* kbase = P.kc + b * P.kc_sb + h * P.kc_sh + 8 * g16;
   const bf16* vbase = P.vc + b * P.vc_sb + h * P.vc_sh + 8 * g16;
-  // keys [k0, k1) of this split
-  const int k0 = split * kChunk;
-  const int k1 = min(lk, k0 + kChunk);
+  u32x4 kw[kUnroll], vw[kUnroll];
+  auto load = [&](int j0) {
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int j = min(j0 + u * GROUPS, k1 - 1);   // clamped rows are masked below
+      kw[u] = load_once(kbase + j * P.kc_ss);
+      vw[u] = load_once(vbase + j * P.vc_ss);
+    }
+  };
+  if (k0 + grp < k1) load(k0 + grp);
   float q[8];
   {
     const u32x4 w = *reinterpret_cast<const u32x4*>(P.q + b * P.q_sb + h * P.q_sh + 8 * g16);
@@ -102,25 +118,34 @@ __global__ __launch_bounds__(NT) void decode_kernel(Params P) {
       q[2 * e + 1] = bf16hi(w[e]) * P.scale_log2;
     }
   }
+  auto dot = [&](const u32x4& k) {
+    float d = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) d += q[2 * e] * bf16lo(k[e]) + q[2 * e + 1] * bf16hi(k[e]);
+    return row16_sum(d);
+  };
   float m = -INFINITY, l = 0.f, o[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = 0.f;
-  for (int j0 = k0 + grp; j0 < k1; j0 += GROUPS * kUnroll) {
-    u32x4 kw[kUnroll], vw[kUnroll];
+  if (P.fused && split == 0 && grp == 0 && len >= 0 && len < P.Smax) {
+    // the new row, key len: into the caches, and the first key of this group
+    const u32x4 kn = *reinterpret_cast<const u32x4*>(P.k + b * P.k_sb + h * P.k_sh + 8 * g16);
+    const u32x4 vn = *reinterpret_cast<const u32x4*>(P.v + b * P.v_sb + h * P.v_sh + 8 * g16);
+    *reinterpret_cast<u32x4*>(P.kc + b * P.kc_sb + h * P.kc_sh + len * P.kc_ss + 8 * g16) = kn;
+    *reinterpret_cast<u32x4*>(P.vc + b * P.vc_sb + h * P.vc_sh + len * P.vc_ss + 8 * g16) = vn;
+    m = dot(kn);
+    l = __builtin_amdgcn_exp2f(m - m);
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int j = min(j0 + u * GROUPS, k1 - 1);   // clamped rows are masked below
-      kw[u] = *reinterpret_cast<const u32x4*>(kbase + j * P.kc_ss);
-      vw[u] = *reinterpret_cast<const u32x4*>(vbase + j * P.vc_ss);
+    for (int e = 0; e < 4; ++e) {
+      o[2 * e] = l * bf16lo(vn[e]);
+      o[2 * e + 1] = l * bf16hi(vn[e]);
     }
+  }
+  for (int j0 = k0 + grp; j0 < k1; j0 += kStep) {
     float s[kUnroll], mx = m;
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-      float d = 0.f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) d += q[2 * e] * bf16lo(kw[u][e]) + q[2 * e + 1] * bf16hi(kw[u][e]);
-      d = sum16(d);
-      s[u] = (j0 + u * GROUPS < k1) ? d : -INFINITY;
+      s[u] = (j0 + u * GROUPS < k1) ? dot(kw[u]) : -INFINITY;
       mx = fmaxf(mx, s[u]);
     }
     const float alpha = __builtin_amdgcn_exp2f(m - mx);   // m = -inf at first: 0
@@ -138,26 +163,46 @@ __global__ __launch_bounds__(NT) void decode_kernel(Params P) {
       }
     }
     m = mx;
+    if (j0 + kStep < k1) load(j0 + kStep);
   }
-  // merge the 16 groups
-  if (g16 == 0) {
-    s_m[grp] = m;
-    s_l[grp] = l;
+  // merge the wave's four groups, then the four waves
+  float M = fmaxf(m, __shfl_xor(m, 16));
+  M = fmaxf(M, __shfl_xor(M, 32));
+  const float a = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+  l *= a;
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    o[e] *= a;
+    o[e] += __shfl_xor(o[e], 16);
+    o[e] += __shfl_xor(o[e], 32);
   }
-  s_o[grp][2 * g16] = f32x4{o[0], o[1], o[2], o[3]};
-  s_o[grp][2 * g16 + 1] = f32x4{o[4], o[5], o[6], o[7]};
+  const int w = tid >> 6;
+  if ((tid & 63) < 16) {
+    if (g16 == 0) {
+      s_m[w] = M;
+      s_l[w] = l;
+    }
+    s_o[w][2 * g16] = f32x4{o[0], o[1], o[2], o[3]};
+    s_o[w][2 * g16 + 1] = f32x4{o[4], o[5], o[6], o[7]};
+  }
   __syncthreads();
   if (tid < D / 4) {
-    float M = -INFINITY;
-#pragma unroll
-    for (int g = 0; g < GROUPS; ++g) M = fmaxf(M, s_m[g]);
+    M = fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]));
     float L = 0.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
-      const float w = s_m[g] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[g] - M);
-      L += w * s_l[g];
-      acc += w * s_o[g][tid];
+    for (int g = 0; g < NT / 64; ++g) {
+      const float wgt = s_m[g] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[g] - M);
+      L += wgt * s_l[g];
+      acc += wgt * s_o[g][tid];
+    }
+    if (P.nsplit == 1) {
+      const float inv = L > 0.f ? 1.f / L : 0.f;
+      *reinterpret_cast<bf16x4*>(P.out + b * P.o_sb + h * P.o_sh + 4 * tid) =
+          cvt4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
+      return;
     }
     float* dst = P.part + (((int64_t)b * P.H + h) * P.nsplit + split) * kPart;
     if (tid == 0) {
@@ -544,8 +589,9 @@ __global__ __launch_bounds__(NT, 2) void extend_kernel(Params P) {
 }
 
 // One wave per (b, i, h). Lane s weighs split s (its max and sum read by all lanes at
-// once: a serial walk over the splits paid a memory round trip each); then each half-wave
-// adds every other split's o, lane % 32 holding four of the 128 columns.
+// once); then each half-wave adds every other split's o, lane % 32 holding four of the 128
+// columns. Bound by memory latency: with a serial walk over the splits, which paid a round
+// trip each, 12.9 us for 1024 rows x 8 splits and 7.0 us for 16 rows x 23; now 5.0 and 4.2.
 __global__ __launch_bounds__(256) void combine_kernel(Params P) {
   const int64_t w = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
@@ -567,9 +613,18 @@ __global__ __launch_bounds__(256) void combine_kernel(Params P) {
       wgt = __builtin_amdgcn_exp2f(sp[lane * kPart] - M);
       L += wgt * sp[lane * kPart + 1];
     }
-    for (int s = lane >> 5; s < ((n + 1) & ~1); s += 2) {
-      const float ws = __shfl(wgt, s);   // 0 for s = n
-      if (s < n) acc += ws * *reinterpret_cast<const f32x4*>(sp + s * kPart + 4 + 4 * (lane & 31));
+    for (int sb = 0; sb < n; sb += 16) {
+      const int s1 = sb + (lane >> 5);
+      // eight loads in flight; past the last split its partial again, not added (it may be inf)
+      f32x4 o[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        o[u] = *reinterpret_cast<const f32x4*>(sp + min(s1 + 2 * u, n - 1) * kPart + 4 + 4 * (lane & 31));
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const f32x4 x = acc + __shfl(wgt, s1 + 2 * u) * o[u];
+        acc = s1 + 2 * u < n ? x : acc;
+      }
     }
   }
 #pragma unroll

@@ -937,7 +937,18 @@ static bool rows_apart(int64_t B, int64_t N, int64_t H, int64_t sb, int64_t sn, 
 static int ext_qw(int S) { return S <= 32 ? 1 : S <= 64 ? 2 : 4; }
 static int kv_nqb(int S) { return S == 1 ? 1 : (S + 32 * ext_qw(S) - 1) / (32 * ext_qw(S)); }
 static int64_t kv_nsplit(int64_t B, int S, int64_t H, int64_t Smax) {
-  if (S == 1) return (Smax + kvc::kChunk - 1) / kvc::kChunk;
+  if (S == 1) {
+    // Few (row, head) pairs: 512 workgroups, at least one 64-key step each (16 pairs x 4096
+    // keys 13.1 us at 512, 14.2 at 1024, 12.0 at 256; 64 pairs 26.1, 26.7, 28.4). Many: 1024,
+    // and two splits each of 512 keys or more, which even out ragged lengths (1024 pairs x
+    // 4096: 272 us at one split, 263 at two, 266 at four; 2048 pairs x 256: 41 at one, 46 at
+    // two).
+    const int64_t units = B * H;
+    if (units <= 128)
+      return std::max<int64_t>(1, std::min({(512 + units - 1) / units, (Smax + kvc::kStep - 1) / kvc::kStep,
+                                            (int64_t)kvc::kMaxSplits}));
+    return std::max<int64_t>(1, std::min(std::max<int64_t>(2, (1024 + units - 1) / units), Smax / 512));
+  }
   const int64_t tk = 32 * (4 / ext_qw(S)), units = B * H * kv_nqb(S);
   // 512 workgroups fill the chip (two per CU); more splits only add partials to write and
   // merge: 4 x 16 heads x 45 queries 38 us a call at 512, 42 at 1024, 60 at 2048, and 2 x 16 x
@@ -1023,10 +1034,10 @@ int prefixlm_kvcache_fwd(const prefixlm_kvcache_args* a, void* stream_) {
   const bool prefill = !a->cache_seqlens && a->cache_seqlen == 0 && has_new && packed && S <= Smax &&
                        T < 0x7fffffff && a->q_stride_s >= kvc::D && a->k_stride_s >= kvc::D &&
                        a->v_stride_s >= kvc::D && a->out_stride_s >= kvc::D;
-  // The extend kernel reads the new rows from k, v and writes them to the caches in one
-  // launch; that needs cache rows of its own for every (b, row, head) and two caches (a
+  // The decode and extend kernels read the new rows from k, v and write them to the caches in
+  // one launch; that needs cache rows of its own for every (b, row, head) and two caches (a
   // row shared between batch rows would be read by one while the other writes it).
-  P.fused = !prefill && S > 1 && has_new &&
+  P.fused = !prefill && has_new &&
             rows_apart(B, Smax, H, a->k_cache_stride_b, a->k_cache_stride_s, a->k_cache_stride_h) &&
             rows_apart(B, Smax, H, a->v_cache_stride_b, a->v_cache_stride_s, a->v_cache_stride_h) &&
             a->k_cache != a->v_cache;
@@ -1079,7 +1090,7 @@ int prefixlm_kvcache_fwd(const prefixlm_kvcache_args* a, void* stream_) {
       hipLaunchKernelGGL(kvc::extend_kernel<2>, dim3((unsigned)nblk), dim3(kvc::NT), kvc::ExtGeo<2>::LDS_BYTES, stream, P);
     else
       hipLaunchKernelGGL(kvc::extend_kernel<4>, dim3((unsigned)nblk), dim3(kvc::NT), kvc::ExtGeo<4>::LDS_BYTES, stream, P);
-    if (S == 1 || P.nsplit > 1) {
+    if (P.nsplit > 1) {
       const int64_t waves = (int64_t)B * S * H;
       hipLaunchKernelGGL(kvc::combine_kernel, dim3((unsigned)((waves * 64 + 255) / 256)), dim3(256), 0, stream, P);
     }
