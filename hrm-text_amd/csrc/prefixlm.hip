@@ -804,8 +804,10 @@ static int swiglu_launch(const prefixlm_swiglu_args* a, void* stream_, bool back
                      a->rows, a->cols};
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
   (void)hipGetLastError();
-  hipLaunchKernelGGL(backward ? nm::swiglu_bwd_kernel : nm::swiglu_fwd_kernel, dim3((unsigned)((threads + 255) / 256)),
-                     dim3(256), 0, stream, P);
+  const bool nt = a->rows * a->cols * (backward ? 10 : 6) > nm::kNtBytes;
+  hipLaunchKernelGGL(backward ? (nt ? nm::swiglu_bwd_kernel<true> : nm::swiglu_bwd_kernel<false>)
+                              : (nt ? nm::swiglu_fwd_kernel<true> : nm::swiglu_fwd_kernel<false>),
+                     dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, P);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(PREFIXLM_ERR_HIP, "swiglu launch: %s", hipGetErrorString(e));
   return PREFIXLM_OK;
