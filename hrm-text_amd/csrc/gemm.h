@@ -13,41 +13,51 @@
 // `rstd` (one fp32 per row, from a row pass before the GEMM), to the fp32 products.
 // With norm off, r = 1. Each output is rounded to bf16 once.
 //
-// Workgroup: 256 x rows by 256 W rows, 8 waves (two per SIMD) of 128 x rows by 64 W rows,
+// Workgroup: MT x rows by 256 W rows, 8 waves (two per SIMD) of MT / 2 x rows by 64 W rows,
 // K in stages of 64 staged by direct global->LDS loads (two stages: the next one lands
 // while this one is read). Every wave computes Y^T tiles (A = W rows, B = x rows; lane =
 // output row, registers = output columns), so a gate tile and its up tile meet in the
 // same lanes and the epilogue stores whole rows.
+//
+// Persistent: one workgroup per CU walks its tiles, and the stages of successive tiles form
+// one stream, so the next tile's first stages load under this tile's last ones and its
+// epilogue (which stages through LDS of its own).
+//
+// Bound by the board's power at large M (a stage takes the same 2700 cycles at any load, at
+// 2.4 GHz for 44 workgroups and about 1.75 with every CU busy), by the fill of the CUs at small
+// M. K 2048, N 11264 with SwiGLU: M 16384 642 us (1.18 PFLOP/s), M 1100 51 us. Before (a
+// workgroup per tile, m tiles dealt to the XCDs by number, a stage's direct loads issued in
+// one burst): 656 and 102 us: five m tiles kept three XCDs idle and gave the others two rounds.
 #pragma once
 #include "common.h"
 
 namespace prefixlm {
 namespace mlp {
 
-constexpr int MT = 256;              // x rows per workgroup
 constexpr int WT = 256;              // W rows per workgroup
 constexpr int KT = 64;               // K per stage (four MFMA k steps between barriers)
-constexpr int NSTAGE = 128 / KT;     // LDS stages (128 KB in all): one in flight while one is read
 constexpr int KS = KT / 16;          // MFMA k steps per stage
 constexpr int NTH = 512;             // 8 waves, two per SIMD
 constexpr int ROWB = KT * 2;         // bytes of one staged row
 constexpr int CPR = ROWB / 16;       // 16-byte chunks per staged row
-constexpr int RPW = 256 / ROWB;      // staged rows per 256-byte bank window
-constexpr int RPB = 1024 / ROWB;     // staged rows per 1 KB direct load
-constexpr int NDMA = 32 / RPB;       // direct loads per wave, operand and stage (32 rows)
-constexpr int A_BYTES = MT * ROWB;   // x tile
-constexpr int B_BYTES = WT * ROWB;   // W tile
-constexpr int STAGE = A_BYTES + B_BYTES;
-constexpr int LDS_BYTES = NSTAGE * STAGE;   // the output staging reuses it
-constexpr int OUT_RS = 64 * 2 + 16;         // output staging row: 64 bf16 + 16 B pad
-static_assert(KS % 2 == 0 && CPR * RPW == 16 && NSTAGE >= 2, "stage geometry");
-static_assert(8 * 32 * OUT_RS <= LDS_BYTES && NDMA >= 1, "output staging fits in LDS");
+constexpr int OUT_ROW = 64 * 2;      // output staging row: 64 bf16, chunks swizzled
 
-// Staged row r, logical 16-byte chunk c lives at r * ROWB + 16 (c ^ f(r)),
-// f(r) = (r / RPW) % CPR: the 16 rows of one quarter-wave operand read (a fixed chunk)
-// land on 16 different 16-byte positions of the 256-byte bank window, so the operand
-// reads are free of bank conflicts.
-__device__ __forceinline__ int swz_f(int r) { return (r / RPW) % CPR; }
+template <int MT>
+struct Geo {
+  static constexpr int MI = MT / 64;             // 32-row x operands per wave
+  static constexpr int NX = MT / 64;             // direct x loads per wave and stage (8 rows each)
+  static constexpr int NW = WT / 64;             // direct W loads per wave and stage
+  static constexpr int A_BYTES = MT * ROWB;      // x tile
+  static constexpr int STAGE = A_BYTES + WT * ROWB;
+  static constexpr int OUT = 2 * STAGE;          // output staging, 32 rows per wave
+  static constexpr int LDS_BYTES = OUT + 8 * 32 * OUT_ROW;
+  static_assert(KS == 4 && CPR == 8 && NX <= NW && LDS_BYTES <= 160 * 1024, "stage geometry");
+};
+
+// Staged row r, logical 16-byte chunk c lives at r * ROWB + 16 (c ^ f(r)), f(r) = (r / 2) % 8:
+// the 16 rows of one quarter-wave operand read (a fixed chunk) land on 16 different 16-byte
+// positions of the 256-byte bank window, so the operand reads are free of bank conflicts.
+__device__ __forceinline__ int swz_f(int r) { return (r >> 1) & 7; }
 
 struct Params {
   const bf16* x;
@@ -59,58 +69,80 @@ struct Params {
   int m_tiles, n_tiles;
 };
 
-template <bool SWIGLU, bool NORM>
+// Tile number -> (m tile, n tile): groups of 8 m tiles, n after n within a group, so the 32
+// consecutive tiles that an XCD's CUs work on together share 8 x slices and 4 W slices in its L2.
+__device__ __forceinline__ void tile_at(const Params& P, int id, int* mt, int* nt) {
+  const int per = 8 * P.n_tiles, g = id / per, r = id - g * per;
+  const int gm = min(8, P.m_tiles - 8 * g);
+  *nt = r / gm;
+  *mt = 8 * g + (r - *nt * gm);
+}
+
+// 16 bytes per lane straight to LDS, lane j at dst + 16 j (dst wave-uniform)
+typedef __attribute__((address_space(3))) char lds_char;
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t rsrc, lds_char* dst, uint32_t voffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)dst, 16, voffset, 0, 0, 0);
+}
+
+template <int MT, bool SWIGLU, bool NORM>
 __global__ __launch_bounds__(NTH, 1) void proj_gemm_kernel(Params P) {
+  using G = Geo<MT>;
+  constexpr int MI = G::MI;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  // XCD-aware order: XCD b % 8 runs the m tiles congruent to it mod 8. Its workgroups
-  // take them in groups of 8 m tiles; within a group, 32 consecutive workgroups (one per
-  // CU of the XCD, running together) cover 8 m tiles x 4 n tiles, so each x slice is
-  // shared by 4 of them and each W slice by 8 in the XCD's L2.
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  const int per_group = 8 * ((P.n_tiles + 3) / 4 * 4);
-  const int grp = j / per_group, r = j - grp * per_group;
-  const int nt = 4 * (r >> 5) + (r & 3);
-  const int mt = xcd + 8 * (8 * grp + ((r & 31) >> 2));
-  if (mt >= P.m_tiles || nt >= P.n_tiles) return;
-  const int m0 = mt * MT;
+  // XCD b % 8 takes a contiguous eighth of the tiles, its workgroups one after another
+  const int total = P.m_tiles * P.n_tiles, xcd = blockIdx.x & 7;
+  const int t_end = (int)((int64_t)(xcd + 1) * total / 8), step = gridDim.x >> 3;
+  int id = (int)((int64_t)xcd * total / 8) + (int)(blockIdx.x >> 3);
+  if (id >= t_end) return;
   const int F = P.N >> 1;
-  // W rows of this tile: SWIGLU: gate rows n0..n0+127 then up rows F+n0..; PLAIN: n0..n0+255
-  const int n0 = nt * (SWIGLU ? WT / 2 : WT);
 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
-  const int wm = w >> 2, wn = w & 3;   // 2 x 4 waves of 128 x rows by 64 W rows
+  const int wm = w >> 2, wn = w & 3;   // 2 x 4 waves
 
-  const __amdgpu_buffer_rsrc_t xr = make_rsrc(P.x + (int64_t)m0 * P.ldx,
-                                              rows_bytes(min(MT, P.M - m0), P.ldx, P.K));
-  const __amdgpu_buffer_rsrc_t wr = make_rsrc(P.w, rows_bytes(P.N, P.ldw, P.K));
-
-  // Direct global -> LDS loads: one instruction moves RPB rows (1 KB); lane L writes
-  // slot L % CPR of row RPB i + L / CPR, which holds logical chunk (L % CPR) ^ f(row).
-  // Wave w loads rows 32 w .. 32 w + 31 of both tiles (NDMA instructions each).
-  uint32_t xoff[NDMA], woff[NDMA];
-  {
-    // W rows of the wave's 32: SWIGLU waves 0-3 the gate rows, 4-7 the up rows
-    const int wbase = SWIGLU ? (w < 4 ? n0 + 32 * w : F + n0 + 32 * (w - 4)) : n0 + 32 * w;
+  // Direct global -> LDS loads: one instruction moves 8 rows (1 KB); lane L writes slot L % 8
+  // of row L / 8, which holds logical chunk (L % 8) ^ f(row). Wave w loads x rows
+  // MT / 8 * w .. and W rows 32 w .. of the tile (SWIGLU: waves 0-3 gate rows, 4-7 up rows).
+  uint32_t xoff[G::NX], woff[G::NW];
 #pragma unroll
-    for (int i = 0; i < NDMA; ++i) {
-      const int tr = 32 * w + RPB * i + lane / CPR;   // tile row
-      const int ch = (lane % CPR) ^ swz_f(tr);
-      xoff[i] = (uint32_t)((int64_t)tr * P.ldx * 2) + ch * 16;
-      woff[i] = (uint32_t)((int64_t)(wbase + RPB * i + lane / CPR) * P.ldw * 2) + ch * 16;
-    }
+  for (int i = 0; i < G::NX; ++i) {
+    const int r = MT / 8 * w + 8 * i + lane / CPR;
+    xoff[i] = (uint32_t)((int64_t)r * P.ldx * 2) + 16 * ((lane % CPR) ^ swz_f(r));
   }
-  typedef __attribute__((address_space(3))) char lds_char;
-  auto issue_stage_at = [&](int buf, int kk) {
-    lds_char* base = (lds_char*)smem + buf * STAGE + 32 * w * ROWB;
-    const uint32_t k2 = (uint32_t)(kk * ROWB);
 #pragma unroll
-    for (int i = 0; i < NDMA; ++i) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(base + 1024 * i), 16,
-                                               xoff[i] + k2, 0, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(base + A_BYTES + 1024 * i),
-                                               16, woff[i] + k2, 0, 0, 0);
+  for (int i = 0; i < G::NW; ++i) {
+    const int r = 32 * w + 8 * i + lane / CPR;
+    const int row = SWIGLU && w >= 4 ? F + r - 128 : r;
+    woff[i] = (uint32_t)((int64_t)row * P.ldw * 2) + 16 * ((lane % CPR) ^ swz_f(r));
+  }
+  const int nk = P.K / KT;
+  int mt, nt;
+  tile_at(P, id, &mt, &nt);
+  // the load cursor: the stage after the last one issued; past the last tile it stays on that
+  // tile's last stage (loads into buffers nobody reads, so that every stage issues the same)
+  int ld_id = id, ld_kk = 0, ld_mt = mt, ld_nt = nt;
+  auto advance = [&]() {
+    if (ld_kk + 1 < nk) {
+      ++ld_kk;
+    } else if (ld_id + step < t_end) {
+      ld_id += step;
+      ld_kk = 0;
+      tile_at(P, ld_id, &ld_mt, &ld_nt);
+    }
+  };
+  // direct loads [lo, hi) of the cursor's stage into buffer buf
+  auto issue = [&](int buf, int lo, int hi) {
+    const uint32_t k2 = (uint32_t)(ld_kk * ROWB);
+    // W rows of n tile nt: from row 128 nt of each half (SWIGLU) or 256 nt on
+    const int m0 = ld_mt * MT, n0 = ld_nt * (SWIGLU ? WT / 2 : WT);
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(P.x + (int64_t)m0 * P.ldx, rows_bytes(min(MT, P.M - m0), P.ldx, P.K));
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(P.w + (int64_t)n0 * P.ldw, rows_bytes(P.N - n0, P.ldw, P.K));
+    lds_char* base = (lds_char*)smem + buf * G::STAGE;
+#pragma unroll
+    for (int i = lo; i < hi; ++i) {
+      if (i < G::NX) load_lds16(xr, base + MT / 8 * w * ROWB + 1024 * i, xoff[i] + k2);
+      load_lds16(wr, base + G::A_BYTES + 32 * w * ROWB + 1024 * i, woff[i] + k2);
     }
   };
 
@@ -123,124 +155,126 @@ __global__ __launch_bounds__(NTH, 1) void proj_gemm_kernel(Params P) {
   // W tile rows of A operand bi: SWIGLU: bi = 0 the gate rows 32 wn, bi = 1 the up rows
   // 128 + 32 wn of the same output columns; PLAIN: 64 wn + 32 bi
   auto a_row = [&](int bi) { return SWIGLU ? bi * (WT / 2) + 32 * wn : 64 * wn + 32 * bi; };
-  const int brow0 = 128 * wm;   // x rows of B operand mi: brow0 + 32 mi
+  const int brow0 = MT / 2 * wm;   // x rows of B operand mi: brow0 + 32 mi
 
-  f32x16 acc[4][2];   // [mi: x rows][bi: W rows]; Y^T tiles (register = W row, lane = x row)
-#pragma unroll
-  for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mi][bi][r] = 0.f;
-
-  const int nk = P.K / KT;
-  // LDS reads of k step ks of stage kk into fragment set `set`
-  bf16x8 af[2][2], bfr[2][4];
-  auto rd = [&](int kk, int ks, int set) {
-    const char* abase = smem + (kk % NSTAGE) * STAGE + A_BYTES + l32 * ROWB + coff[ks];
-    const char* bbase = smem + (kk % NSTAGE) * STAGE + l32 * ROWB + coff[ks];
+  f32x16 acc[MI][2];   // [mi: x rows][bi: W rows]; Y^T tiles (register = W row, lane = x row)
+  // LDS reads of k step ks of buffer buf into fragment set `set`
+  bf16x8 af[2][2], bfr[2][MI];
+  auto rd = [&](int buf, int ks, int set) {
+    const char* abase = smem + buf * G::STAGE + G::A_BYTES + l32 * ROWB + coff[ks];
+    const char* bbase = smem + buf * G::STAGE + l32 * ROWB + coff[ks];
 #pragma unroll
     for (int i = 0; i < 2; ++i) af[set][i] = *reinterpret_cast<const bf16x8*>(abase + a_row(i) * ROWB);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) bfr[set][i] = *reinterpret_cast<const bf16x8*>(bbase + (brow0 + 32 * i) * ROWB);
+    for (int i = 0; i < MI; ++i) bfr[set][i] = *reinterpret_cast<const bf16x8*>(bbase + (brow0 + 32 * i) * ROWB);
   };
-  // MFMAs of x operands mi in [m_lo, m_hi) of fragment set `set`
-  auto mm_part = [&](int set, int m_lo, int m_hi) {
+  auto mm = [&](int set, int mi) {
 #pragma unroll
-    for (int mi = m_lo; mi < m_hi; ++mi)
-#pragma unroll
-      for (int bi = 0; bi < 2; ++bi) acc[mi][bi] = mfma32x32x16(af[set][bi], bfr[set][mi], acc[mi][bi]);
+    for (int bi = 0; bi < 2; ++bi) acc[mi][bi] = mfma32x32x16(af[set][bi], bfr[set][mi], acc[mi][bi]);
   };
-  // Stage loads past the last stage re-read the last one into a buffer nobody reads
-  // again, so every stage has the same loads in flight and the loop body has no branch
-  // (a branch would let the compiler sink the reads below the MFMAs they should overlap
-  // and make it wait for all of them).
-  auto issue = [&](int kk) { issue_stage_at(kk % NSTAGE, min(kk, nk - 1)); };
-  // waits until this wave's loads of the oldest stage in flight are in LDS (the
-  // NSTAGE - 2 younger stages stay in flight), then a plain barrier (no memory fence:
-  // it would also wait for the younger stages)
+  // waits until this wave's loads of the stage in flight are in LDS, then a plain barrier
+  // (the workgroup fence of __syncthreads would also wait for the output stores)
   auto stage_barrier = [&]() {
     sched_fence();
-    waitcnt<2 * NDMA * (NSTAGE - 2), 0>();
+    waitcnt<0, 0>();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     sched_fence();
   };
-#pragma unroll
-  for (int s = 0; s < NSTAGE - 1; ++s) issue(s);
+
+  // In the last k step of a stage, after its first MFMAs, the next stage is waited for, the
+  // workgroup syncs, and the buffer of this stage (every wave's reads of it are done) takes
+  // the stage after: half of its direct loads between this step's MFMAs and half between
+  // those of the next stage's first step. All of them at once, before the operand reads, kept
+  // the matrix cores idle while eight waves issued 64 KB.
+  constexpr int HALF = G::NW / 2;
+  issue(0, 0, G::NW);
+  advance();
   stage_barrier();   // stage 0 in LDS
-  issue(NSTAGE - 1);
+  issue(1, 0, HALF);
   rd(0, 0, 0);
-  // Stage kk: k steps 0 .. KS-1, each step's MFMAs running over the next step's reads.
-  // In the last step, after the first MFMAs, stage kk + 1 is waited for, the workgroup
-  // syncs, stage kk + NSTAGE is issued into the buffer of stage kk (every wave's reads of
-  // it are done), and the reads of stage kk + 1's first step run under the remaining
-  // MFMAs. (Each step's first MFMAs come before the next reads are issued, so the wait
-  // for their operands does not also wait for the reads issued after them.)
-  for (int kk = 0; kk < nk; ++kk) {
+  int buf = 0;
+  for (;;) {
+    const int m0 = mt * MT;
+    float rs[MI];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int set = ks & 1;
-      sched_fence();
-      mm_part(set, 0, 1);
-      sched_fence();
-      if (ks + 1 < KS) {
-        rd(kk, ks + 1, set ^ 1);
-      } else if (kk + 1 < nk) {
-        stage_barrier();
-        issue(kk + NSTAGE);
-        rd(kk + 1, 0, set ^ 1);
-      }
-      sched_fence();
-      mm_part(set, 1, 4);
+    for (int mi = 0; mi < MI; ++mi) {
+      rs[mi] = NORM ? P.rstd[min(m0 + brow0 + 32 * mi + l32, P.M - 1)] : 1.f;
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mi][bi][r] = 0.f;
     }
+    for (int kk = 0; kk < nk; ++kk) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int set = ks & 1;
+        sched_fence();
+        mm(set, 0);
+        sched_fence();
+        if (ks + 1 < KS) {
+          rd(buf, ks + 1, set ^ 1);
+        } else {
+          stage_barrier();
+          advance();
+          rd(buf ^ 1, 0, set ^ 1);
+        }
+#pragma unroll
+        for (int m = 1; m < MI; ++m) {
+          sched_fence();
+          if (m <= HALF) {
+            constexpr int PER = MI - 1 < HALF ? HALF : 1;   // loads per slot (MT 128: one slot)
+            if (ks == KS - 1) issue(buf, PER * (m - 1), PER * m);
+            if (ks == 0) issue(buf ^ 1, HALF + PER * (m - 1), HALF + PER * m);
+          }
+          sched_fence();
+          mm(set, m);
+        }
+      }
+      buf ^= 1;
+    }
+    // ---- epilogue ----------------------------------------------------------------
+    // 32 rows at a time through the wave's own LDS (chunk c of row r at c ^ (r % 8)), stored
+    // as whole rows of the wave's columns: 32 (SWIGLU) or 64
+    char* wl = smem + G::OUT + w * 32 * OUT_ROW;
+    constexpr int NOT = SWIGLU ? 1 : 2;                      // output 32-column tiles of the wave
+    constexpr int CPO = 4 * NOT, RPP = 64 / CPO;             // 16-byte chunks per row, rows per pass
+    const int ycol0 = SWIGLU ? nt * (WT / 2) + 32 * wn : nt * WT + 64 * wn;
+    const __amdgpu_buffer_rsrc_t yr = make_rsrc(P.y + (int64_t)m0 * P.ldy,
+                                                rows_bytes(min(MT, P.M - m0), P.ldy, SWIGLU ? F : P.N));
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi) {
+      // lane holds columns 8 (reg / 4) + 4 hh + reg % 4 of each 32-column tile
+#pragma unroll
+      for (int ti = 0; ti < NOT; ++ti)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float o[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (SWIGLU) {
+              const float g = acc[mi][0][4 * q + e] * rs[mi], u = acc[mi][1][4 * q + e] * rs[mi];
+              o[e] = g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-g * kLog2e)) * u;
+            } else {
+              o[e] = acc[mi][ti][4 * q + e] * rs[mi];
+            }
+          }
+          *reinterpret_cast<bf16x4*>(wl + l32 * OUT_ROW + (((4 * ti + q) ^ (l32 & 7)) * 16) + 8 * hh) =
+              cvt4(o[0], o[1], o[2], o[3]);
+        }
+#pragma unroll
+      for (int k = 0; k < 32 / RPP; ++k) {
+        const int rr = lane / CPO + RPP * k, ch = lane % CPO;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(wl + rr * OUT_ROW + ((ch ^ (rr & 7)) * 16));
+        buf_store16(v, yr, (uint32_t)((int64_t)(brow0 + 32 * mi + rr) * P.ldy * 2) + (uint32_t)(ycol0 * 2 + ch * 16));
+      }
+    }
+    id += step;
+    if (id >= t_end) break;
+    tile_at(P, id, &mt, &nt);
   }
   waitcnt<0, 15>();   // no stage load left in flight
-  __syncthreads();
-
-  // ---- epilogue ------------------------------------------------------------------
-  float r4[4];
-#pragma unroll
-  for (int mi = 0; mi < 4; ++mi) {
-    const int row = min(m0 + brow0 + 32 * mi + l32, P.M - 1);
-    r4[mi] = NORM ? P.rstd[row] : 1.f;
-  }
-  char* wl = smem + w * 32 * OUT_RS;
-  constexpr int NOT = SWIGLU ? 1 : 2;                      // output 32-column tiles of the wave
-  const int ycol0 = SWIGLU ? nt * (WT / 2) + 32 * wn : n0 + 64 * wn;
-  const __amdgpu_buffer_rsrc_t yr = make_rsrc(P.y + (int64_t)m0 * P.ldy,
-                                              rows_bytes(min(MT, P.M - m0), P.ldy, SWIGLU ? F : P.N));
-#pragma unroll
-  for (int mi = 0; mi < 4; ++mi) {
-    const float r = r4[mi];
-    // lane holds columns 8 (reg / 4) + 4 hh + reg % 4 of each 32-column tile
-#pragma unroll
-    for (int ti = 0; ti < NOT; ++ti)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (SWIGLU) {
-            const float g = acc[mi][0][4 * q + e] * r, u = acc[mi][1][4 * q + e] * r;
-            o[e] = g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-g * kLog2e)) * u;
-          } else {
-            o[e] = acc[mi][ti][4 * q + e] * r;
-          }
-        }
-        *reinterpret_cast<bf16x4*>(wl + l32 * OUT_RS + (32 * ti + 8 * q + 4 * hh) * 2) = cvt4(o[0], o[1], o[2], o[3]);
-      }
-    // 32 rows x 32 NOT columns: chunk (lane % CPO) of row (lane / CPO) + RPP k
-    constexpr int CPO = 32 * NOT / 8;                      // 16-byte chunks per output row
-    constexpr int RPP = 64 / CPO;                          // rows per pass
-#pragma unroll
-    for (int k = 0; k < 32 / RPP; ++k) {
-      const int rr = lane / CPO + RPP * k, ch = lane % CPO;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(wl + rr * OUT_RS + ch * 16);
-      buf_store16(v, yr, (uint32_t)((int64_t)(brow0 + 32 * mi + rr) * P.ldy * 2) + (uint32_t)(ycol0 * 2 + ch * 16));
-    }
-  }
 }
 
 }  // namespace mlp

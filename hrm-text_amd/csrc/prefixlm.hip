@@ -885,26 +885,38 @@ int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
     if (a->K > nm::kNormMaxCols) return fail(PREFIXLM_ERR_INVALID, "norm: K=%d exceeds %d", a->K, nm::kNormMaxCols);
   }
   // 32-bit byte offsets: within a 256-row tile of x and y, and over all of W
-  if ((int64_t)mlp::MT * a->x_stride * 2 >= ((int64_t)1 << 31) ||
-      (int64_t)mlp::MT * a->y_stride * 2 >= ((int64_t)1 << 31) || (int64_t)a->N * a->w_stride * 2 >= ((int64_t)1 << 32))
+  if ((int64_t)256 * a->x_stride * 2 >= ((int64_t)1 << 31) ||
+      (int64_t)256 * a->y_stride * 2 >= ((int64_t)1 << 31) || (int64_t)a->N * a->w_stride * 2 >= ((int64_t)1 << 32))
     return fail(PREFIXLM_ERR_INVALID, "operands exceed the 32-bit offsets of the kernel");
-  static std::once_flag once;
-  static hipError_t attr_err = hipSuccess;
-  void (*const kernels[4])(mlp::Params) = {mlp::proj_gemm_kernel<false, false>, mlp::proj_gemm_kernel<false, true>,
-                                           mlp::proj_gemm_kernel<true, false>, mlp::proj_gemm_kernel<true, true>};
-  std::call_once(once, [&kernels] {
-    for (int i = 0; i < 4 && attr_err == hipSuccess; ++i)
-      attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernels[i]),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, mlp::LDS_BYTES);
-  });
-  if (attr_err != hipSuccess) return fail(PREFIXLM_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
+  int cus = 0;
+  const int rc = persistent_grid(&cus);
+  if (rc) return rc;
   mlp::Params P{static_cast<const bf16*>(a->x), static_cast<const bf16*>(a->w), static_cast<bf16*>(a->y),
                 a->rstd, a->x_stride, a->w_stride, a->y_stride, a->M, a->K, a->N, 0, 0};
-  P.m_tiles = (a->M + mlp::MT - 1) / mlp::MT;
-  P.n_tiles = (int)(sw ? a->N / mlp::WT : a->N / mlp::WT);
-  // per XCD: groups of 8 m tiles, each over the n tiles in blocks of 4 (see the kernel)
-  const int64_t grid = 8 * (int64_t)((P.m_tiles + 63) / 64) * 8 * ((P.n_tiles + 3) / 4 * 4);
-  if (grid > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "grid too large");
+  P.n_tiles = a->N / mlp::WT;
+  // 256 x rows per tile, or 128 where that needs fewer or shorter rounds over the CUs: a round
+  // of 128-row tiles takes 0.65 (many rounds) to 0.8 (one) of a round of 256-row ones, the W
+  // tile's loads staying the same (K 2048, N 11264: M 512 34 us with 128 rows, 44 with 256;
+  // M 700 65 and 45; M 1100 70 and 51; M 16384 832 and 642)
+  const int64_t t256 = (int64_t)((a->M + 255) / 256) * P.n_tiles, t128 = (int64_t)((a->M + 127) / 128) * P.n_tiles;
+  if (t128 > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "grid too large");
+  const bool half = 7 * ((t128 + cus - 1) / cus) < 10 * ((t256 + cus - 1) / cus);
+  P.m_tiles = (a->M + (half ? 127 : 255)) / (half ? 128 : 256);
+  const int tiles = (int)(half ? t128 : t256);
+  const unsigned grid = (unsigned)std::min(cus, (tiles + 7) / 8 * 8);
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  void (*const kernels[8])(mlp::Params) = {
+      mlp::proj_gemm_kernel<256, false, false>, mlp::proj_gemm_kernel<256, false, true>,
+      mlp::proj_gemm_kernel<256, true, false>,  mlp::proj_gemm_kernel<256, true, true>,
+      mlp::proj_gemm_kernel<128, false, false>, mlp::proj_gemm_kernel<128, false, true>,
+      mlp::proj_gemm_kernel<128, true, false>,  mlp::proj_gemm_kernel<128, true, true>};
+  std::call_once(once, [&kernels] {
+    for (int i = 0; i < 8 && attr_err == hipSuccess; ++i)
+      attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernels[i]), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     i < 4 ? mlp::Geo<256>::LDS_BYTES : mlp::Geo<128>::LDS_BYTES);
+  });
+  if (attr_err != hipSuccess) return fail(PREFIXLM_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
   (void)hipGetLastError();
   if (a->norm) {
@@ -913,8 +925,8 @@ int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
                      a->M, a->K, a->eps};
     hipLaunchKernelGGL(rmsnorm_kernel(a->K, false), dim3((unsigned)((a->M + 3) / 4)), dim3(256), 0, stream, N);
   }
-  hipLaunchKernelGGL(kernels[2 * (sw ? 1 : 0) + (a->norm ? 1 : 0)], dim3((unsigned)grid), dim3(mlp::NTH),
-                     mlp::LDS_BYTES, stream, P);
+  hipLaunchKernelGGL(kernels[4 * (half ? 1 : 0) + 2 * (sw ? 1 : 0) + (a->norm ? 1 : 0)], dim3(grid), dim3(mlp::NTH),
+                     half ? mlp::Geo<128>::LDS_BYTES : mlp::Geo<256>::LDS_BYTES, stream, P);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(PREFIXLM_ERR_HIP, "projection gemm launch: %s", hipGetErrorString(e));
   return PREFIXLM_OK;
