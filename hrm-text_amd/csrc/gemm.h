@@ -10,7 +10,8 @@
 // (Nout = N, or F for SWIGLU). The weightless RMSNorm is a per-row scale,
 // rmsnorm(x) W^T = diag(r) (x W^T) with r = (mean(x^2) + eps)^(-1/2), so the kernel
 // multiplies x's raw rows (never writing the normalized x) and applies r, read from
-// `rstd` (one fp32 per row, from a row pass before the GEMM), to the fp32 products.
+// `rstd` (one fp32 per row, from a row pass before the GEMM; the kernel for few rows computes
+// and writes it itself), to the fp32 products.
 // With norm off, r = 1. Each output is rounded to bf16 once.
 //
 // Workgroup: MT x rows by 256 W rows, 8 waves (two per SIMD) of MT / 2 x rows by 64 W rows,
@@ -275,6 +276,153 @@ __global__ __launch_bounds__(NTH, 1) void proj_gemm_kernel(Params P) {
     tile_at(P, id, &mt, &nt);
   }
   waitcnt<0, 15>();   // no stage load left in flight
+}
+
+// ---- few rows (M <= 128) ---------------------------------------------------------------
+// The product is then a stream of W: a workgroup takes 32 of its rows (SWIGLU: 32 gate rows
+// and the 32 up rows of the same columns) and all x rows, its NWV waves taking K blocks of 64 in
+// turn; both operands go from global memory straight into MFMA fragments (a W row's 128
+// bytes of a block are one line, read by four loads back to back; x stays in L2), and the
+// waves' partial products meet in LDS, wave v finishing two (NWV = 8) or four register rows
+// of every tile. The row scales come from the x fragments on the way, so the norm needs no
+// launch of its own.
+// Bound by the stream of W up to 32 rows, by the repeated reads of x from L2 above: K 2048,
+// N 11264 (46 MB) 11.5 us for 1 row and 12.8 for 16 (4 TB/s), 18.7 for 64, 24.5 for 100; the
+// 128-row tiles take 32 us for any of them (44 workgroups), which x reads would reach past
+// 128 rows.
+template <int MB, int NWV>
+struct SkinnyGeo {
+  static constexpr int TILE = 64 * 16 * 4;       // one wave's partial 32 x 32 tile
+  static constexpr int lds(bool swiglu) { return NWV * (swiglu ? 2 : 1) * MB * TILE + NWV * MB * 32 * 4; }
+};
+
+template <int MB, int NWV, bool SWIGLU, bool NORM>
+__global__ __launch_bounds__(64 * NWV, 1) void proj_skinny_kernel(Params P, float* rstd_out, float eps) {
+  constexpr int NB = SWIGLU ? 2 : 1, RW = 16 / NWV;   // W operands; register rows a wave finishes
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+  const int n0 = blockIdx.x * 32, F = P.N >> 1;
+  const bf16* wp[NB];
+  const bf16* xp[MB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) wp[i] = P.w + (int64_t)(n0 + i * F + l32) * P.ldw + 8 * hh;
+#pragma unroll
+  for (int i = 0; i < MB; ++i) xp[i] = P.x + (int64_t)min(32 * i + l32, P.M - 1) * P.ldx + 8 * hh;
+
+  f32x16 acc[NB][MB];
+  float ss[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    ss[m] = 0.f;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][m][r] = 0.f;
+  }
+  u32x4 wf[2][NB][4], xf[2][MB][4];
+  auto load = [&](int set, int b) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) wf[set][i][s] = *reinterpret_cast<const u32x4*>(wp[i] + 64 * b + 16 * s);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) xf[set][i][s] = *reinterpret_cast<const u32x4*>(xp[i] + 64 * b + 16 * s);
+  };
+  auto mul = [&](int set) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        if (NORM) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float a = bf16lo(xf[set][m][s][e]), b = bf16hi(xf[set][m][s][e]);
+            ss[m] += a * a;
+            ss[m] += b * b;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+          acc[i][m] = mfma32x32x16(__builtin_bit_cast(bf16x8, wf[set][i][s]), __builtin_bit_cast(bf16x8, xf[set][m][s]),
+                                   acc[i][m]);
+      }
+  };
+  const int nb = P.K / KT;
+  if (w < nb) load(0, w);
+  for (int b = w; b < nb; b += 2 * NWV) {
+    if (b + NWV < nb) load(1, b + NWV);
+    mul(0);
+    if (b + NWV < nb) {
+      if (b + 2 * NWV < nb) load(0, b + 2 * NWV);
+      mul(1);
+    }
+  }
+  // partial tiles: [wave][operand][m][register / 4][lane] of 16 bytes, then the sums of squares
+  float* sums = reinterpret_cast<float*>(smem + NWV * NB * MB * SkinnyGeo<MB, NWV>::TILE);
+  auto part = [&](int v, int i, int m, int r4) {
+    return reinterpret_cast<f32x4*>(smem) + ((((v * NB + i) * MB + m) * 4 + r4) * 64 + lane);
+  };
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4)
+        *part(w, i, m, r4) = f32x4{acc[i][m][4 * r4], acc[i][m][4 * r4 + 1], acc[i][m][4 * r4 + 2], acc[i][m][4 * r4 + 3]};
+    if (NORM) {
+      const float s = halves_sum(ss[m]);
+      if (hh == 0) sums[(w * MB + m) * 32 + l32] = s;
+    }
+  }
+  __syncthreads();
+  // wave w: registers RW w .. RW w + RW - 1, i.e. columns 8 (r / 4) + 4 hh + r % 4
+  const int r0 = RW * w;
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    const int row = 32 * m + l32;
+    float rs = 1.f;
+    if (NORM) {
+      float s = 0.f;
+#pragma unroll
+      for (int v = 0; v < NWV; ++v) s += sums[(v * MB + m) * 32 + l32];
+      rs = __builtin_amdgcn_rsqf(s / (float)P.K + eps);
+      if (blockIdx.x == 0 && w == 0 && hh == 0 && row < P.M) rstd_out[row] = rs;
+    }
+    float t[NB][RW];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int e = 0; e < RW; ++e) t[i][e] = 0.f;
+#pragma unroll
+    for (int v = 0; v < NWV; ++v)
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const float* p = reinterpret_cast<const float*>(part(v, i, m, r0 >> 2)) + (r0 & 3);
+#pragma unroll
+        for (int e = 0; e < RW; ++e) t[i][e] += p[e];
+      }
+    float o[RW];
+#pragma unroll
+    for (int e = 0; e < RW; ++e) {
+      if (SWIGLU) {
+        const float g = t[0][e] * rs, u = t[NB - 1][e] * rs;
+        o[e] = g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-g * kLog2e)) * u;
+      } else {
+        o[e] = t[0][e] * rs;
+      }
+    }
+    if (row < P.M) {
+      bf16* yp = P.y + (int64_t)row * P.ldy + n0 + 8 * (r0 >> 2) + 4 * hh + (r0 & 3);
+      if (RW == 4)
+        *reinterpret_cast<bf16x4*>(yp) = cvt4(o[0], o[1], o[RW - 2], o[RW - 1]);
+      else
+        *reinterpret_cast<uint32_t*>(yp) = __builtin_bit_cast(u32x2, cvt4(o[0], o[1], 0.f, 0.f))[0];
+    }
+  }
 }
 
 }  // namespace mlp

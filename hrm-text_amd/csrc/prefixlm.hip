@@ -864,6 +864,40 @@ static int rmsnorm_launch(const prefixlm_rmsnorm_args* a, void* stream_, bool ba
 int prefixlm_rmsnorm_fwd(const prefixlm_rmsnorm_args* a, void* stream) { return rmsnorm_launch(a, stream, false); }
 int prefixlm_rmsnorm_bwd(const prefixlm_rmsnorm_args* a, void* stream) { return rmsnorm_launch(a, stream, true); }
 
+}  // extern "C"
+
+// Projections of at most 128 rows: the kernel that streams W (see gemm.h).
+template <int MB, int NWV>
+static int proj_skinny_launch(const mlp::Params& P, bool sw, bool norm, float* rstd, float eps, hipStream_t stream) {
+  using Kernel = void (*)(mlp::Params, float*, float);
+  using G = mlp::SkinnyGeo<MB, NWV>;
+  const Kernel kernels[4] = {mlp::proj_skinny_kernel<MB, NWV, false, false>, mlp::proj_skinny_kernel<MB, NWV, false, true>,
+                             mlp::proj_skinny_kernel<MB, NWV, true, false>, mlp::proj_skinny_kernel<MB, NWV, true, true>};
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  std::call_once(once, [&kernels] {
+    for (int i = 0; i < 4 && attr_err == hipSuccess; ++i)
+      attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernels[i]), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     G::lds(i >= 2));
+  });
+  if (attr_err != hipSuccess) return fail(PREFIXLM_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
+  hipLaunchKernelGGL(kernels[2 * (sw ? 1 : 0) + (norm ? 1 : 0)], dim3((unsigned)((sw ? P.N / 2 : P.N) / 32)), dim3(64 * NWV),
+                     G::lds(sw), stream, P, rstd, eps);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(PREFIXLM_ERR_HIP, "projection launch: %s", hipGetErrorString(e));
+  return PREFIXLM_OK;
+}
+static int proj_skinny(const prefixlm_proj_gemm_args* a, hipStream_t stream) {
+  const mlp::Params P{static_cast<const bf16*>(a->x), static_cast<const bf16*>(a->w), static_cast<bf16*>(a->y),
+                      nullptr, a->x_stride, a->w_stride, a->y_stride, a->M, a->K, a->N, 0, 0};
+  const bool sw = a->swiglu != 0, norm = a->norm != 0;
+  if (a->M <= 32) return proj_skinny_launch<1, 8>(P, sw, norm, a->rstd, a->eps, stream);
+  if (a->M <= 64) return proj_skinny_launch<2, 8>(P, sw, norm, a->rstd, a->eps, stream);
+  return proj_skinny_launch<4, 4>(P, sw, norm, a->rstd, a->eps, stream);
+}
+
+extern "C" {
+
 int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
   if (!a) return fail(PREFIXLM_ERR_INVALID, "args is null");
   const bool sw = a->swiglu != 0;
@@ -888,6 +922,9 @@ int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
   if ((int64_t)256 * a->x_stride * 2 >= ((int64_t)1 << 31) ||
       (int64_t)256 * a->y_stride * 2 >= ((int64_t)1 << 31) || (int64_t)a->N * a->w_stride * 2 >= ((int64_t)1 << 32))
     return fail(PREFIXLM_ERR_INVALID, "operands exceed the 32-bit offsets of the kernel");
+  hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+  (void)hipGetLastError();
+  if (a->M <= 128) return proj_skinny(a, stream);
   int cus = 0;
   const int rc = persistent_grid(&cus);
   if (rc) return rc;
@@ -917,8 +954,6 @@ int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
                                      i < 4 ? mlp::Geo<256>::LDS_BYTES : mlp::Geo<128>::LDS_BYTES);
   });
   if (attr_err != hipSuccess) return fail(PREFIXLM_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
-  hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-  (void)hipGetLastError();
   if (a->norm) {
     // the row scales first (a wave per row, x read once; the normalized x is not written)
     nm::NormParams N{static_cast<const bf16*>(a->x), nullptr, nullptr, nullptr, a->rstd, a->x_stride, 0, 0, 0,
