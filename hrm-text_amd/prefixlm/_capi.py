@@ -216,6 +216,13 @@ class Timer:
     launch is bracketed by HIP events on its stream."""
 
     _active = None
+    on_change = None   # called with the active timer's handle (None: none): the native host path
+
+    @classmethod
+    def _set(cls, timer):
+        Timer._active = timer
+        if Timer.on_change is not None:
+            Timer.on_change(timer._h if timer is not None else None)
 
     def __init__(self):
         self._h = load().prefixlm_timer_create()
@@ -223,11 +230,11 @@ class Timer:
             raise RuntimeError("prefixlm_timer_create failed")
 
     def __enter__(self):
-        Timer._active = self
+        Timer._set(self)
         return self
 
     def __exit__(self, *exc):
-        Timer._active = None
+        Timer._set(None)
 
     def read(self):
         """{kernel name: (total_ms, launches)} since the last read (synchronizes)."""

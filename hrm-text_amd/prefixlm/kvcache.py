@@ -29,7 +29,7 @@ import torch
 from torch import Tensor
 
 from . import _capi
-from .op import _ptr, _stream
+from .op import _native_calls, _ptr, _stream
 
 __all__ = ["flash_attn_with_kvcache", "kvcache_attn"]
 
@@ -104,10 +104,15 @@ def flash_attn_with_kvcache(q: Tensor, k_cache: Tensor, v_cache: Tensor, k: Opti
     if used:
         raise NotImplementedError(f"flash_attn_with_kvcache: unsupported arguments {sorted(used)}")
     del num_splits
-    if softmax_scale is None:
-        softmax_scale = 1.0 / math.sqrt(q.shape[-1])
     if cache_seqlens is None:
         cache_seqlens = 0
+    native = _native_calls()
+    if native is not None:
+        out = native.kvcache(q, k_cache, v_cache, k, v, cache_seqlens, softmax_scale, causal)
+        if out is not None:
+            return out
+    if softmax_scale is None:
+        softmax_scale = 1.0 / math.sqrt(q.shape[-1])
     if isinstance(cache_seqlens, int):
         return kvcache_attn(q, k, v, k_cache, v_cache, None, cache_seqlens, bool(causal), float(softmax_scale))
     return kvcache_attn(q, k, v, k_cache, v_cache, cache_seqlens, 0, bool(causal), float(softmax_scale))

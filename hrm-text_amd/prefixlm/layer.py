@@ -32,7 +32,7 @@ from torch import Tensor
 
 from . import _capi
 from .op import (_as_cpu_scalar_tensor, _check_lists_after_launch, _check_plan_before_launch, _check_q_amax,
-                 _cpu_scalar, _ds_arg, _ds_blocks_arg, _meta, _plan_arg, _ptr, _q_amax_count, _stream)
+                 _cpu_scalar, _ds_arg, _ds_blocks_arg, _meta, _native_calls, _plan_arg, _ptr, _q_amax_count, _stream)
 
 __all__ = ["fused_attention_layer", "FusedAttentionLayer", "rope", "attn_layer_fwd", "attn_layer_bwd"]
 
@@ -225,6 +225,12 @@ def fused_attention_layer(gqkv: Tensor, cos: Tensor, sin: Tensor, is_causal: boo
     models/layers.py:135) and the gathered cos, sin [T, 128] fp32. Returns
     [T, H, 128] bf16; reshape to [T, H*128] for the output projection. ``plan`` and
     ``plan_ds_blocks`` as in ``flash_attn_varlen_prefixlm``."""
+    native = _native_calls()
+    if native is not None:
+        y = native.layer(gqkv, cos, sin, is_causal, prefix_lens, causal_lens, cu_seqlens, total_seqlen, numseqs,
+                         max_seqlen_prefix, max_seqlen_causal, max_seqlen_all, softmax_scale, plan, plan_ds_blocks)
+        if y is not None:
+            return y
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(gqkv.shape[-1])
     scal = [_as_cpu_scalar_tensor(x) for x in

@@ -21,7 +21,7 @@ import torch
 from torch import Tensor
 
 from . import _capi
-from .op import _ptr, _stream
+from .op import _native_calls, _ptr, _stream
 
 __all__ = ["swiglu", "rms_norm", "swiglu_fwd", "swiglu_bwd", "rms_norm_fwd", "rms_norm_bwd", "proj_gemm",
            "rms_norm_linear", "rms_norm_swiglu"]
@@ -92,7 +92,9 @@ class SwiGLUFunction(torch.autograd.Function):
 
 def swiglu(gu: Tensor) -> Tensor:
     """``F.silu(gate) * up`` with ``gate, up = gu.chunk(2, dim=-1)`` (models/layers.py:167-168)."""
-    return SwiGLUFunction.apply(gu)
+    native = _native_calls()
+    y = native.swiglu(gu) if native is not None else None
+    return SwiGLUFunction.apply(gu) if y is None else y
 
 
 @torch.library.custom_op("prefixlm::rms_norm_fwd", mutates_args=())
@@ -153,7 +155,9 @@ class RMSNormFunction(torch.autograd.Function):
 
 def rms_norm(x: Tensor, eps: float = 1e-6) -> Tensor:
     """``F.rms_norm(x, (x.shape[-1],), eps=eps)`` without a weight (models/transformer.py:87)."""
-    return RMSNormFunction.apply(x, eps)
+    native = _native_calls()
+    y = native.rms_norm(x, eps) if native is not None else None
+    return RMSNormFunction.apply(x, eps) if y is None else y
 
 
 # ---- projections with the norm and the SwiGLU fused in (forward only) ------------------
@@ -187,6 +191,12 @@ def _proj_gemm_fake(x, w, swiglu, norm, eps):
     return x.new_empty((*x.shape[:-1], n))
 
 
+def _proj(x: Tensor, w: Tensor, swiglu: bool, eps: float) -> Tensor:
+    native = _native_calls()
+    y = native.proj_gemm(x, w, swiglu, True, eps) if native is not None else None
+    return proj_gemm(x, w, swiglu, True, eps) if y is None else y
+
+
 def rms_norm_linear(x: Tensor, w: Tensor, eps: float) -> Tensor:
     """F.linear(F.rms_norm(x, (K,), eps), w) in one GEMM (forward only).
 
@@ -194,7 +204,7 @@ def rms_norm_linear(x: Tensor, w: Tensor, eps: float) -> Tensor:
     the config-5 shapes against 1.44 for hipBLASLt, so at 2048 -> 8192 columns the norm
     kernel plus the library GEMM is faster (0.38 vs 0.48 ms). Kept for callers that
     want the normalized activations never written."""
-    return proj_gemm(x, w, False, True, float(eps))
+    return _proj(x, w, False, float(eps))
 
 
 def rms_norm_swiglu(x: Tensor, w_gate_up: Tensor, eps: float) -> Tensor:
@@ -204,4 +214,4 @@ def rms_norm_swiglu(x: Tensor, w_gate_up: Tensor, eps: float) -> Tensor:
     Not recommended for speed: it saves the two elementwise passes but its GEMM core is
     slower than hipBLASLt's (about 1.22 vs 1.44 PFLOP/s), which cancels the saving inside
     the config-5 stack (150.5 vs 149.6 ms per step with and without it)."""
-    return proj_gemm(x, w_gate_up, True, True, float(eps))
+    return _proj(x, w_gate_up, True, float(eps))

@@ -38,7 +38,7 @@ from typing import Optional, Tuple
 import torch
 from torch import Tensor
 
-from . import _capi
+from . import _capi, _native
 
 __all__ = ["flash_attn_varlen_prefixlm", "FlashAttnVarlenPrefixLM", "varlen_fwd", "varlen_bwd"]
 
@@ -359,6 +359,14 @@ class FlashAttnVarlenPrefixLM(torch.autograd.Function):
         return dq, dk, dv, *((None,) * 12)
 
 
+def _native_calls():
+    """The native host path for this call, or None: while a compiler traces, or in checking
+    mode, the Python path runs."""
+    if torch.compiler.is_compiling() or _CHECK_METADATA:
+        return None
+    return _native.calls()
+
+
 def _as_cpu_scalar_tensor(x) -> Tensor:
     if isinstance(x, Tensor):
         return x
@@ -384,6 +392,13 @@ def flash_attn_varlen_prefixlm(q: Tensor, k: Tensor, v: Tensor, is_causal: bool,
     ``prefixlm.plan.plan_ds_blocks`` as a CPU scalar, which sizes the backward's dS
     buffer exactly (``prefixlm.plan.plan_inputs`` returns both).
     """
+    native = _native_calls()
+    if native is not None:
+        out = native.varlen(q, k, v, is_causal, prefix_lens, causal_lens, cu_seqlens, total_seqlen, numseqs,
+                            max_seqlen_prefix, max_seqlen_causal, max_seqlen_all, softmax_scale, plan,
+                            plan_ds_blocks)
+        if out is not None:
+            return out
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(q.shape[-1])
     scal = [_as_cpu_scalar_tensor(x) for x in

@@ -1,0 +1,152 @@
+"""GPU: the native host path of the public calls against the Python path they replace:
+bitwise the same results and gradients, the same refusals, and the calls it hands back
+(operands that need a copy, recorded and batched backwards, modes, saved-tensor hooks)."""
+import pytest
+import torch
+
+from prefixlm import (_native, flash_attn_varlen_prefixlm, flash_attn_with_kvcache, fused_attention_layer, plan_inputs,
+                      rms_norm, swiglu)
+from prefixlm.hrm_stack import rotary_cos_sin
+from prefixlm.norm_mlp import rms_norm_linear, rms_norm_swiglu
+from prefixlm.synth import make_batch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+@pytest.fixture(params=["native", "python"])
+def path(request, monkeypatch):
+    assert _native.calls() is not None, "the native host path is not built"
+    if request.param == "python":
+        monkeypatch.setattr(_native, "_module", None)
+    return request.param
+
+
+def _rand(*shape, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16).to(DEV)
+
+
+def _both(fn, monkeypatch):
+    """fn's results on the native and on the Python path."""
+    assert _native.calls() is not None
+    a = fn()
+    with monkeypatch.context() as m:
+        m.setattr(_native, "_module", None)
+        b = fn()
+    for x, y in zip(a, b):
+        assert x.dtype == y.dtype and torch.equal(x, y)
+
+
+@pytest.mark.parametrize("plan", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("ints", [False, True])
+def test_varlen_bitwise(plan, D, ints, monkeypatch):
+    b = make_batch([10, 130, 0], [40, 7, 90], 300, 4, D, seed=5, device=DEV)
+    info = dict(b.seq_info)
+    if plan:
+        info.update(plan_inputs(b.seq_tensors, b.seq_scalars, DEV))
+    if ints:
+        info = {k: int(x) if isinstance(x, torch.Tensor) and x.dim() == 0 else x for k, x in info.items()}
+
+    def run():
+        q, k = (t.clone().requires_grad_() for t in (b.q, b.k))
+        v = torch.stack((b.v, b.v), 1)[:, 1].requires_grad_()        # a strided view
+        out = flash_attn_varlen_prefixlm(q, k, v, False, **info)
+        g = torch.autograd.grad(out, (q, k, v), b.dout, retain_graph=True)
+        g2 = torch.autograd.grad(out.float().sum(), (q, k, v))       # an expanded gradient
+        with torch.no_grad():
+            o = flash_attn_varlen_prefixlm(q, k, v, True, **info)
+        return out, *g, *g2, o
+    _both(run, monkeypatch)
+
+
+def test_layer_norm_activation_projection_bitwise(monkeypatch):
+    T, H = 260, 2
+    b = make_batch([60, 20], [100, 70], T, H, 128, seed=6, device=DEV, with_dout=False)
+    cos, sin = rotary_cos_sin(torch.arange(T, device=DEV), 128, 10000.0, 1024)
+    gq, dy = _rand(T, 4 * H, 128, seed=1), _rand(T, H, 128, seed=2)
+    x, gu, w = _rand(7, 9, 256, seed=3), _rand(40, 512, seed=4), _rand(512, 256, seed=5)
+
+    def run():
+        g = gq.clone().requires_grad_()
+        y = fused_attention_layer(g, cos, sin, False, **b.seq_info)
+        xx, uu = x.clone().requires_grad_(), gu.clone().requires_grad_()
+        n, a = rms_norm(xx, 1e-6), swiglu(uu)
+        grads = torch.autograd.grad((y, n, a), (g, xx, uu), (dy, x, a.detach()))
+        with torch.no_grad():
+            return (y, n, a, *grads, rms_norm(x[:, ::2], 1e-5), swiglu(gu), rms_norm_linear(x, torch.nn.Parameter(w), 1e-6),
+                    rms_norm_swiglu(x.view(63, 256)[:, :256], w, 1e-6))
+    _both(run, monkeypatch)
+
+
+@pytest.mark.parametrize("S", [1, 5])
+def test_kvcache_bitwise_and_in_place(S, monkeypatch):
+    B, H, Smax = 2, 3, 150
+    q, k, v = (_rand(B, S, H, 128, seed=i) for i in range(3))
+    caches = _rand(2, B, Smax, H, 128, seed=9)
+    lens = torch.tensor([20, 140], dtype=torch.int32, device=DEV)
+
+    def run():
+        kc, vc = caches[0].clone(), caches[1].clone()
+        before = kc._version, vc._version
+        o = flash_attn_with_kvcache(q, kc, vc, k=k, v=v, cache_seqlens=lens, causal=True)
+        assert (kc._version, vc._version) == tuple(n + 1 for n in before)
+        o2 = flash_attn_with_kvcache(q, kc, vc, cache_seqlens=30)
+        return o, kc, vc, o2
+    _both(run, monkeypatch)
+
+
+def test_refusals(path):
+    b = make_batch([10], [40], 64, 2, 128, seed=5, device=DEV)
+    with pytest.raises(TypeError):
+        flash_attn_varlen_prefixlm(b.q.float(), b.k, b.v, False, **b.seq_info)
+    with pytest.raises(ValueError):
+        flash_attn_varlen_prefixlm(b.q, b.k[:32], b.v, False, **b.seq_info)
+    with pytest.raises(AssertionError):
+        flash_attn_varlen_prefixlm(b.q, b.k, b.v, False, **{**b.seq_info, "numseqs": torch.tensor(1, device=DEV)})
+    with pytest.raises(RuntimeError, match="total_seqlen"):
+        flash_attn_varlen_prefixlm(b.q, b.k, b.v, False, **{**b.seq_info, "total_seqlen": torch.tensor(65)})
+    with pytest.raises(RuntimeError, match="multiple"):
+        rms_norm(_rand(4, 12), 1e-6)
+    with pytest.raises(ValueError):
+        swiglu(_rand(4, 24))
+    q = b.q.clone().requires_grad_()
+    out = flash_attn_varlen_prefixlm(q, b.k, b.v, False, **b.seq_info)
+    with torch.no_grad():
+        q.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+
+
+def test_recorded_backward_is_the_custom_op(path):
+    """create_graph: the gradient carries a graph whose own backward is refused."""
+    b = make_batch([10], [40], 64, 2, 128, seed=5, device=DEV)
+    q = b.q.clone().requires_grad_()
+    out = flash_attn_varlen_prefixlm(q, b.k, b.v, False, **b.seq_info)
+    (g,) = torch.autograd.grad(out, q, b.dout.clone().requires_grad_(), create_graph=True)
+    assert g.requires_grad
+    with pytest.raises(RuntimeError):
+        g.float().sum().backward()
+
+
+def test_hooks_checkpoint_and_other_streams(path):
+    b = make_batch([10, 30], [40, 20], 128, 2, 128, seed=5, device=DEV)
+    q = b.q.clone().requires_grad_()
+    f = lambda q: flash_attn_varlen_prefixlm(q, b.k, b.v, False, **b.seq_info)  # noqa: E731
+    want, = torch.autograd.grad(f(q), q, b.dout)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t.clone(), lambda t: t):
+        out = f(q)
+    assert torch.equal(torch.autograd.grad(out, q, b.dout)[0], want) and len(packed) >= 7
+    out = torch.utils.checkpoint.checkpoint(f, q, use_reentrant=False)
+    assert torch.equal(torch.autograd.grad(out, q, b.dout)[0], want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        out = f(q)
+        got, = torch.autograd.grad(out, q, b.dout)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    with torch.inference_mode():
+        assert torch.equal(f(q.detach()), out.detach())
