@@ -1125,7 +1125,7 @@ __global__ __launch_bounds__(q2::NT, 3) void prefixlm_bwd_dq_ds_kernel(Q2Params 
 // =====================================================================================
 // pre-pass and padding rows
 // =====================================================================================
-constexpr int kPreRows = 32;     // token rows per pre-pass workgroup
+constexpr int kPreRows = 32;     // token rows per pre-pass workgroup, at most (see pre_rows)
 constexpr int kPreBatch = 8;     // row-heads per 16-lane group whose loads are in flight together
 constexpr int kPreMaxHeads = 64; // per-head maxima kept in LDS
 
@@ -1150,16 +1150,37 @@ struct GateBwd {
   int64_t g_st, g_sh, dg_st, dg_sh, da_st, da_sh;
 };
 
+// dq = dk = dv = 0 on the rows past total, which no other kernel of the backward writes: by the
+// pre-pass workgroups of those rows
+struct PadBwd {
+  bf16* dq;
+  bf16* dk;
+  bf16* dv;
+  int64_t dq_st, dq_sh, dk_st, dk_sh, dv_st, dv_sh;
+};
+template <int HD>
+__device__ __forceinline__ void zero_gradients(const PadBwd& G, int64_t t0, int64_t t1, int H) {
+  constexpr int CPR = HD / 8;   // 16-byte chunks per (row, head)
+  const u32x4 z = {0u, 0u, 0u, 0u};
+  for (int64_t t = t0; t < t1; ++t)
+    for (int idx = threadIdx.x; idx < H * CPR; idx += 256) {
+      const int h = idx / CPR, chunk = idx % CPR;
+      *reinterpret_cast<u32x4*>(G.dq + t * G.dq_st + h * G.dq_sh + chunk * 8) = z;
+      *reinterpret_cast<u32x4*>(G.dk + t * G.dk_st + h * G.dk_sh + chunk * 8) = z;
+      *reinterpret_cast<u32x4*>(G.dv + t * G.dv_st + h * G.dv_sh + chunk * 8) = z;
+    }
+}
+
 template <int HD, bool GATED>
 __global__ __launch_bounds__(256) void prefixlm_bwd_pre_kernel(
     const bf16* o, const int8_t* o_lo, const bf16* dout, int64_t o_st, int64_t o_sh, int64_t lo_st,
     int64_t lo_sh, int64_t do_st, int64_t do_sh, float* delta, float* stats, int T, int H, int total,
-    GateBwd G, const float* q_amax, int q_slots) {
+    GateBwd G, const float* q_amax, int q_slots, PadBwd pad, int rows_per_wg) {
   static_assert(HD == 128 || !GATED, "the output gate is applied at head dim 128");
   constexpr int D = HD, NW = HD / 32;   // 32-bit words (bf16 pairs) per lane
   __shared__ int smax[kPreMaxHeads * kStats];
-  const int t0 = blockIdx.x * kPreRows;
-  const int rows = min(kPreRows, T - t0);
+  const int t0 = blockIdx.x * rows_per_wg;
+  const int rows = min(rows_per_wg, T - t0);
   const int tid = threadIdx.x;
   const int grp = tid >> 4, chunk = tid & 15;
   for (int i = tid; i < H * kStats; i += 256) smax[i] = 0;
@@ -1171,6 +1192,7 @@ __global__ __launch_bounds__(256) void prefixlm_bwd_pre_kernel(
   const float qv = q_own ? q_amax[qb] : 0.f;
   __syncthreads();
   const int vrows = max(0, min(rows, total - t0));   // rows of this range below total
+  if (vrows < rows) zero_gradients<HD>(pad, t0 + vrows, t0 + rows, H);
   const __amdgpu_buffer_rsrc_t orr = make_rsrc(o + t0 * o_st, rows_bytes(vrows, o_st, (int)((H - 1) * o_sh + D)));
   const __amdgpu_buffer_rsrc_t lor =
       make_rsrc(o_lo ? static_cast<const void*>(o_lo + t0 * lo_st) : o,
@@ -1299,22 +1321,6 @@ __global__ __launch_bounds__(256) void prefixlm_bwd_pre_kernel(
   __syncthreads();
   for (int i = tid; i < H * kStats; i += 256) {
     if (smax[i] != 0) atomicMax(reinterpret_cast<int*>(stats + i), smax[i]);
-  }
-}
-
-// dq = dk = dv = 0 on rows total .. T-1 (one workgroup per row)
-template <int HD>
-__global__ __launch_bounds__(256) void prefixlm_bwd_pad_kernel(bf16* dq, bf16* dk, bf16* dv, int64_t dq_st,
-                                                               int64_t dq_sh, int64_t dk_st, int64_t dk_sh,
-                                                               int64_t dv_st, int64_t dv_sh, int H, int total) {
-  constexpr int CPR = HD / 8;   // 16-byte chunks per (row, head)
-  const int64_t t = total + (int64_t)blockIdx.x;
-  const u32x4 z = {0u, 0u, 0u, 0u};
-  for (int idx = threadIdx.x; idx < H * CPR; idx += 256) {
-    const int h = idx / CPR, chunk = idx % CPR;
-    *reinterpret_cast<u32x4*>(dq + t * dq_st + h * dq_sh + chunk * 8) = z;
-    *reinterpret_cast<u32x4*>(dk + t * dk_st + h * dk_sh + chunk * 8) = z;
-    *reinterpret_cast<u32x4*>(dv + t * dv_st + h * dv_sh + chunk * 8) = z;
   }
 }
 

@@ -75,36 +75,99 @@ struct Params {
   int T, H, is_causal;
   int numseqs;       // items naming a segment >= numseqs (a stale plan) are skipped
   float scale_log2;  // softmax_scale * log2(e)
+  // grid indices from n_main on: the rows past total_seqlen (or, in a prefill, the append),
+  // by workgroups of their own that need no other launch and run beside the last items
+  int n_main, total;
+  // UNIFORM (a prefill of numseqs sequences of seq_len new rows each): no work list and no
+  // metadata; the new rows of k and v also go to the caches
+  int seq_len;
+  bf16* kc;
+  bf16* vc;
+  int64_t kc_sb, kc_ss, kc_sh, vc_sb, vc_ss, vc_sh;
 };
+
+// Rows >= total_seqlen: out = 0 (with its residual and the gated output) and lse = -inf
+// (reference :130; FA3 leaves its LSE there unspecified). An HD / 8-thread group per (row,
+// head), 16 B of O (8 elements, and their 8 residual bytes) per thread.
+template <int HD>
+__device__ __forceinline__ void pad_rows(const Params& P, int blk) {
+  constexpr int CPR = HD / 8, GROUPS = NT / CPR;
+  const int64_t gidx = (int64_t)blk * GROUPS + (threadIdx.x / CPR);
+  if (gidx >= (int64_t)(P.T - P.total) * P.H) return;
+  const int t = P.total + (int)(gidx / P.H);
+  const int h = (int)(gidx % P.H);
+  const int chunk = threadIdx.x % CPR;
+  const u32x4 z = {0u, 0u, 0u, 0u};
+  *reinterpret_cast<u32x4*>(P.o + t * P.o_st + h * P.o_sh + chunk * 8) = z;
+  if (P.o_lo) *reinterpret_cast<u32x2*>(P.o_lo + t * P.lo_st + h * P.lo_sh + chunk * 8) = u32x2{0u, 0u};
+  if (P.y) *reinterpret_cast<u32x4*>(P.y + t * P.y_st + h * P.y_sh + chunk * 8) = z;
+  if (chunk == 0) P.lse[(int64_t)h * P.T + t] = -INFINITY;
+}
+// The prefill's append: 16-byte chunks of the new k and v rows, kAppend per thread.
+constexpr int kAppend = 4;
+__device__ __forceinline__ void append_rows(const Params& P, int blk) {
+#pragma unroll
+  for (int u = 0; u < kAppend; ++u) {
+    const int64_t gid = ((int64_t)blk * kAppend + u) * NT + threadIdx.x;
+    const int c = (int)(gid & 15);
+    const int64_t r = gid >> 4;
+    if (r >= (int64_t)P.T * P.H) return;
+    const int64_t t = r / P.H;
+    const int h = (int)(r - t * P.H), b = (int)(t / P.seq_len), i = (int)(t - (int64_t)b * P.seq_len);
+    *reinterpret_cast<u32x4*>(P.kc + b * P.kc_sb + i * P.kc_ss + h * P.kc_sh + 8 * c) =
+        *reinterpret_cast<const u32x4*>(P.k + t * P.k_st + h * P.k_sh + 8 * c);
+    *reinterpret_cast<u32x4*>(P.vc + b * P.vc_sb + i * P.vc_ss + h * P.vc_sh + 8 * c) =
+        *reinterpret_cast<const u32x4*>(P.v + t * P.v_st + h * P.v_sh + 8 * c);
+  }
+}
 
 // Three workgroups per CU at HD = 128 (12 waves, at most 168 VGPRs each): 32-key tiles
 // keep the registers and the LDS (4 tiles of 9.5 KB per workgroup) within that budget,
 // and the third workgroup hides more of each wave's MFMA -> softmax -> MFMA latency
 // than the larger tiles of two workgroups did. HD = 64 halves the Q and O registers
 // and the tiles, and runs four workgroups per CU.
-template <int HD>
+template <int HD, bool UNIFORM = false>
 __global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Params P) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using G = Geo<HD>;
   constexpr int RS = G::RS, TILE = G::TILE, SROWS = G::SROWS, SPASS = G::SPASS, OFF_K = G::OFF_K,
                 OFF_V = G::OFF_V, NS = G::NS, NDT = G::NDT, D = HD;
 
-  int item, h;
-  // a workgroup without work still writes its max |Q| slots (0), so that every slot of
-  // the grid holds a value
-  if (!unit_of(blockIdx.x, P.hdr->n_items, P.H, &item, &h)) {
-    if (P.q_amax != nullptr && threadIdx.x < NT / 64) P.q_amax[NT / 64 * blockIdx.x + threadIdx.x] = 0.f;
+  if ((int)blockIdx.x >= P.n_main) {
+    if constexpr (UNIFORM)
+      append_rows(P, (int)blockIdx.x - P.n_main);
+    else
+      pad_rows<HD>(P, (int)blockIdx.x - P.n_main);
     return;
   }
-  const int2 it = P.items[item];
-  const int seg = it.x, qt = it.y;
-  if (seg < 0 || seg >= P.numseqs) {
-    if (P.q_amax != nullptr && threadIdx.x < NT / 64) P.q_amax[NT / 64 * blockIdx.x + threadIdx.x] = 0.f;
-    return;
+  int item, h, seg, qt, cs, L, p;
+  if constexpr (UNIFORM) {
+    // the last tiles first: with a causal mask they see the most keys
+    const int tiles = (P.seq_len + BM - 1) / BM;
+    if (!unit_of(blockIdx.x, P.numseqs * tiles, P.H, &item, &h)) return;
+    const int back = item / P.numseqs;
+    qt = tiles - 1 - back;
+    seg = item - back * P.numseqs;
+    cs = seg * P.seq_len;
+    L = P.seq_len;
+    p = P.is_causal ? 0 : L;
+  } else {
+    // a workgroup without work still writes its max |Q| slots (0), so that every slot of
+    // the grid holds a value
+    if (!unit_of(blockIdx.x, P.hdr->n_items, P.H, &item, &h)) {
+      if (P.q_amax != nullptr && threadIdx.x < NT / 64) P.q_amax[NT / 64 * blockIdx.x + threadIdx.x] = 0.f;
+      return;
+    }
+    const int2 it = P.items[item];
+    seg = it.x, qt = it.y;
+    if (seg < 0 || seg >= P.numseqs) {
+      if (P.q_amax != nullptr && threadIdx.x < NT / 64) P.q_amax[NT / 64 * blockIdx.x + threadIdx.x] = 0.f;
+      return;
+    }
+    cs = P.cu[seg];
+    L = P.prefix[seg] + P.causal[seg];
+    p = P.is_causal ? 0 : P.prefix[seg];
   }
-  const int cs = P.cu[seg];
-  const int L = P.prefix[seg] + P.causal[seg];
-  const int p = P.is_causal ? 0 : P.prefix[seg];
 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -172,7 +235,7 @@ __global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Para
   for (int s = 0; s < NS; ++s) settle(__builtin_bit_cast(u32x4, qf[s]));
   // max |Q| of the wave's rows, for the backward's fp16 scale of Q (rows past the segment
   // read as 0): bf16 magnitudes compare as 16-bit integers, two per word
-  if (P.q_amax != nullptr) {
+  if (!UNIFORM && P.q_amax != nullptr) {
     u16x2 m = {0, 0};
 #pragma unroll
     for (int s = 0; s < NS; ++s)
@@ -288,7 +351,7 @@ __global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Para
     char* wl = smem + w * out_wave_bytes<NDT>();
     const __amdgpu_buffer_rsrc_t orr = make_rsrc(P.o + cs * P.o_st + h * P.o_sh, rows_bytes(L, P.o_st, D));
     bool gated = false;
-    if constexpr (HD == 128) {
+    if constexpr (HD == 128 && !UNIFORM) {
       if (P.gate != nullptr) {
         const __amdgpu_buffer_rsrc_t gr = make_rsrc(P.gate + cs * P.g_st + h * P.g_sh, rows_bytes(L, P.g_st, D));
         const __amdgpu_buffer_rsrc_t yr = make_rsrc(P.y + cs * P.y_st + h * P.y_sh, rows_bytes(L, P.y_st, D));
@@ -299,36 +362,14 @@ __global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Para
     }
     // O and its residual are read again only by the backward: non-temporal stores
     if (!gated) store_rows_via_lds<NDT, 2>(oacc, inv, wl, orr, qw0, (uint32_t)P.o_st * 2, lane);
-    if (P.o_lo != nullptr) {
+    if (!UNIFORM && P.o_lo != nullptr) {
       // the residual of the rounding above, from the same fp32 values, as int8 codes
       const __amdgpu_buffer_rsrc_t lor =
           make_rsrc(P.o_lo + cs * P.lo_st + h * P.lo_sh, rows_bytes(L, P.lo_st, D, 1));
       store_lo_rows_via_lds<NDT, 2>(oacc, inv, wl, lor, qw0, (uint32_t)P.lo_st, lane);
     }
   }
-  if (wave_active && hh == 0 && qi < L) P.lse[(int64_t)h * P.T + cs + qi] = (m_run + __builtin_log2f(lt)) * kLn2;
-}
-
-// Rows >= total_seqlen: out = 0 (and its residual) and lse = -inf (reference :130;
-// FA3 leaves its LSE there unspecified). One HD/8-thread group per (row, head), 16 B
-// of O (8 elements, and their 8 residual bytes) per thread.
-template <int HD>
-__global__ __launch_bounds__(256) void prefixlm_fwd_pad_kernel(bf16* o, int8_t* o_lo, bf16* y, float* lse,
-                                                                int64_t o_st, int64_t o_sh,
-                                                                int64_t lo_st, int64_t lo_sh, int64_t y_st,
-                                                                int64_t y_sh, int T, int H, int total) {
-  constexpr int CPR = HD / 8, GROUPS = 256 / CPR;
-  const int64_t gidx = (int64_t)blockIdx.x * GROUPS + (threadIdx.x / CPR);
-  const int64_t rows = (int64_t)(T - total) * H;
-  if (gidx >= rows) return;
-  const int t = total + (int)(gidx / H);
-  const int h = (int)(gidx % H);
-  const int chunk = threadIdx.x % CPR;
-  u32x4 z = {0u, 0u, 0u, 0u};
-  *reinterpret_cast<u32x4*>(o + t * o_st + h * o_sh + chunk * 8) = z;
-  if (o_lo) *reinterpret_cast<u32x2*>(o_lo + t * lo_st + h * lo_sh + chunk * 8) = u32x2{0u, 0u};
-  if (y) *reinterpret_cast<u32x4*>(y + t * y_st + h * y_sh + chunk * 8) = z;
-  if (chunk == 0) lse[(int64_t)h * T + t] = -INFINITY;
+  if (!UNIFORM && wave_active && hh == 0 && qi < L) P.lse[(int64_t)h * P.T + cs + qi] = (m_run + __builtin_log2f(lt)) * kLn2;
 }
 
 }  // namespace fwd

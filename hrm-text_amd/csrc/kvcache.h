@@ -10,7 +10,8 @@
 // segment structure: a cache row is one sequence.
 //
 // Kernels:
-//   append  : copies the new k, v rows into the caches (rows past Smax are dropped);
+//   append  : copies the new k, v rows into the caches (rows past Smax are dropped), where the
+//             kernels below do not (see P.fused);
 //   decode  : one query per row, split-K over the keys. A workgroup = (b, h, split); each
 //             16-lane group owns one key at a time (16 x 16-byte chunks of a 256-byte row),
 //             four keys per step, with an online softmax in fp32; the 16 groups are merged
@@ -635,18 +636,6 @@ __global__ __launch_bounds__(256) void combine_kernel(Params P) {
   if (lane < 32)
     *reinterpret_cast<bf16x4*>(P.out + b * P.o_sb + i * P.o_ss + h * P.o_sh + 4 * lane) =
         cvt4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
-}
-
-// metadata of a batched prefill (cache_seqlen 0): batch row b is segment b of S
-// rows, a whole prefix (bidirectional) or, with causal, a whole suffix
-__global__ void prefill_meta_kernel(int32_t* prefix, int32_t* causal_lens, int32_t* cu, int B, int S, int causal) {
-  for (int b = threadIdx.x; b <= B; b += blockDim.x) {
-    if (b < B) {
-      prefix[b] = causal ? 0 : S;
-      causal_lens[b] = causal ? S : 0;
-    }
-    cu[b] = b * S;
-  }
 }
 
 }  // namespace kvc
