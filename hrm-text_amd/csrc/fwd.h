@@ -91,7 +91,8 @@ struct Params {
 // head), 16 B of O (8 elements, and their 8 residual bytes) per thread.
 template <int HD>
 __device__ __forceinline__ void pad_rows(const Params& P, int blk) {
-  constexpr int CPR = HD / 8, GROUPS = NT / CPR;
+  constexpr int CPR = HD / 8;
+  const int GROUPS = blockDim.x / CPR;
   const int64_t gidx = (int64_t)blk * GROUPS + (threadIdx.x / CPR);
   if (gidx >= (int64_t)(P.T - P.total) * P.H) return;
   const int t = P.total + (int)(gidx / P.H);
@@ -108,7 +109,7 @@ constexpr int kAppend = 4;
 __device__ __forceinline__ void append_rows(const Params& P, int blk) {
 #pragma unroll
   for (int u = 0; u < kAppend; ++u) {
-    const int64_t gid = ((int64_t)blk * kAppend + u) * NT + threadIdx.x;
+    const int64_t gid = ((int64_t)blk * kAppend + u) * blockDim.x + threadIdx.x;
     const int c = (int)(gid & 15);
     const int64_t r = gid >> 4;
     if (r >= (int64_t)P.T * P.H) return;
@@ -126,9 +127,16 @@ __device__ __forceinline__ void append_rows(const Params& P, int blk) {
 // and the third workgroup hides more of each wave's MFMA -> softmax -> MFMA latency
 // than the larger tiles of two workgroups did. HD = 64 halves the Q and O registers
 // and the tiles, and runs four workgroups per CU.
-template <int HD, bool UNIFORM = false>
-__global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Params P) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+//
+// KS = 2 (two waves per SIMD in one workgroup, for grids that leave the CUs one workgroup or
+// none): the key tiles are dealt to KS groups of four waves, each with its own LDS tiles and
+// softmax state, and group 0 merges them at the end. A lone wave per SIMD runs its MFMA -> softmax
+// -> MFMA chain at about 1 us per key tile; two share the SIMD at 0.6 us per tile (the softmax's
+// VALU work then bounds it). 2 x 1021 rows x 16 heads (256 workgroups) 32.7 -> 29.7 us a call, 700
+// tokens x 8 heads x d64 the kernel 11.9 -> 10.8 us.
+template <int HD, bool UNIFORM = false, int KS = 1>
+__global__ __launch_bounds__(NT * KS, KS > 1 ? 2 : HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Params P) {
+  extern __shared__ __attribute__((aligned(16))) char smem_all[];
   using G = Geo<HD>;
   constexpr int RS = G::RS, TILE = G::TILE, SROWS = G::SROWS, SPASS = G::SPASS, OFF_K = G::OFF_K,
                 OFF_V = G::OFF_V, NS = G::NS, NDT = G::NDT, D = HD;
@@ -169,7 +177,10 @@ __global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Para
     p = P.is_causal ? 0 : P.prefix[seg];
   }
 
-  const int tid = threadIdx.x;
+  // key group g, and the thread and LDS tiles within it
+  const int g = KS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT) : 0;
+  const int tid = KS > 1 ? (int)threadIdx.x % NT : (int)threadIdx.x;
+  char* const smem = smem_all + g * G::LDS_BYTES;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int q0 = qt * BM;
@@ -206,7 +217,7 @@ __global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Para
       *reinterpret_cast<u32x4*>(stage_base + OFF_V + b * TILE + SROWS * r * RS) = vs[r];
     }
   };
-  if (nk > 0) load_kv(0);
+  if (nk > 0) load_kv(g * BN);
 
   // Q^T fragments: lane holds query qw0+l32, d = 16*s + 8*hh + 0..7
   bf16x8 qf[NS];
@@ -235,7 +246,7 @@ __global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Para
   for (int s = 0; s < NS; ++s) settle(__builtin_bit_cast(u32x4, qf[s]));
   // max |Q| of the wave's rows, for the backward's fp16 scale of Q (rows past the segment
   // read as 0): bf16 magnitudes compare as 16-bit integers, two per word
-  if (!UNIFORM && P.q_amax != nullptr) {
+  if (!UNIFORM && P.q_amax != nullptr && g == 0) {
     u16x2 m = {0, 0};
 #pragma unroll
     for (int s = 0; s < NS; ++s)
@@ -252,10 +263,10 @@ __global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Para
   }
   __syncthreads();
 
-  for (int j = 0; j < nk; ++j) {
+  for (int j = 0; j < (KS > 1 ? (nk + KS - 1) / KS : nk); ++j) {
     const int B = j & 1;
-    const int k0 = j * BN;
-    load_kv(k0 + BN);   // unconditional: the tile past the end goes to a buffer no wave reads again
+    const int k0 = (KS * j + g) * BN;
+    load_kv(k0 + KS * BN);   // unconditional: the tile past the end goes to a buffer no wave reads again
     if (wave_active && k0 < kend_w) {
       // ---- S^T = K Q^T, K rows two steps ahead of the MFMAs -------------------------
       f32x16 sacc[BN / 32];
@@ -345,10 +356,40 @@ __global__ __launch_bounds__(NT, HD == 64 ? 4 : 3) void prefixlm_fwd_kernel(Para
 
   // ---- epilogue: O and its residual as whole rows through LDS, then the LSE ------------
   if (nk == 0) __syncthreads();
-  const float lt = halves_sum(l_run);
+  float lt = halves_sum(l_run);
+  constexpr int MERGE = NDT * 4096 + 512;   // one wave's O (lane-linear), max and sum
+  static_assert(KS <= 2 && (KS == 1 || NT / 64 * MERGE <= KS * G::LDS_BYTES), "the merge area fits in the tiles' LDS");
+  if constexpr (KS > 1) {
+    float* area = reinterpret_cast<float*>(smem_all + w * MERGE);
+    if (g > 0) {
+#pragma unroll
+      for (int t = 0; t < NDT; ++t)
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+          *reinterpret_cast<f32x4*>(area + ((4 * t + m) * 64 + lane) * 4) =
+              f32x4{oacc[t][4 * m], oacc[t][4 * m + 1], oacc[t][4 * m + 2], oacc[t][4 * m + 3]};
+      area[NDT * 1024 + lane] = m_run;
+      area[NDT * 1024 + 64 + lane] = lt;
+    }
+    __syncthreads();
+    if (g > 0) return;
+    const float m1 = area[NDT * 1024 + lane], l1 = area[NDT * 1024 + 64 + lane], M = fmaxf(m_run, m1);
+    const float a0 = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - M);
+    const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - M);
+    m_run = M;
+    lt = a0 * lt + a1 * l1;
+#pragma unroll
+    for (int t = 0; t < NDT; ++t)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(area + ((4 * t + m) * 64 + lane) * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) oacc[t][4 * m + e] = a0 * oacc[t][4 * m + e] + a1 * x[e];
+      }
+  }
   const float inv = wave_active ? 1.f / lt : 0.f;
   {
-    char* wl = smem + w * out_wave_bytes<NDT>();
+    char* wl = smem_all + w * (KS > 1 ? MERGE : out_wave_bytes<NDT>());   // this wave's own area
     const __amdgpu_buffer_rsrc_t orr = make_rsrc(P.o + cs * P.o_st + h * P.o_sh, rows_bytes(L, P.o_st, D));
     bool gated = false;
     if constexpr (HD == 128 && !UNIFORM) {

@@ -151,6 +151,15 @@ void set_kernel_attrs() {
       g_attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd::prefixlm_fwd_kernel<128, true>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, fwd::Geo<128>::LDS_BYTES);
     if (g_attr_err == hipSuccess)
+      g_attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd::prefixlm_fwd_kernel<128, true, 2>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 2 * fwd::Geo<128>::LDS_BYTES);
+    if (g_attr_err == hipSuccess)
+      g_attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd::prefixlm_fwd_kernel<128, false, 2>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 2 * fwd::Geo<128>::LDS_BYTES);
+    if (g_attr_err == hipSuccess)
+      g_attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd::prefixlm_fwd_kernel<64, false, 2>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 2 * fwd::Geo<64>::LDS_BYTES);
+    if (g_attr_err == hipSuccess)
       g_attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&kvc::extend_kernel<1>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kvc::ExtGeo<1>::LDS_BYTES);
     if (g_attr_err == hipSuccess)
@@ -181,6 +190,16 @@ int persistent_grid(int* out) {
   }
   *out = g_cu_count[dev];
   return PREFIXLM_OK;
+}
+
+// Whether the forward deals each item's key tiles to two groups of waves: its grid leaves every
+// CU one workgroup at most, and the segments are long enough (8 key tiles) for half the tiles to
+// outweigh the merge.
+int fwd_splits_keys(int64_t grid, int32_t max_all, bool* split) {
+  int cus = 0;
+  const int rc = persistent_grid(&cus);
+  *split = grid <= cus && max_all >= 8 * fwd::BN;
+  return rc;
 }
 
 // Checks shared by forward and backward. `strides` lists (stride_t, stride_h) pairs.
@@ -392,16 +411,24 @@ static int fwd_launch(const prefixlm_fwd_args* a, void* stream_) {
     P.is_causal = a->is_causal ? 1 : 0;
     P.numseqs = a->numseqs;
     P.scale_log2 = a->softmax_scale * kLog2e;
-    constexpr int groups = fwd::NT / (HD / 8);   // padding (row, head) pairs per workgroup
-    const int64_t nblk = unit_grid(nmax, H), npad = ((int64_t)(T - a->total_seqlen) * H + groups - 1) / groups;
+    const int64_t nblk = unit_grid(nmax, H);
+    bool split = false;
+    rc = fwd_splits_keys(nblk, a->max_seqlen_all, &split);
+    if (rc) return rc;
+    const int nt = fwd::NT * (split ? 2 : 1), groups = nt / (HD / 8);   // padding (row, head) pairs per workgroup
+    const int64_t npad = ((int64_t)(T - a->total_seqlen) * H + groups - 1) / groups;
     if (nblk + npad > 0x7fffffff)
       return fail(PREFIXLM_ERR_INVALID, "grid of %lld blocks too large", (long long)(nblk + npad));
     P.n_main = (int)nblk;
     P.total = a->total_seqlen;
     {
       KernelTimer tm(a->timer, 1, stream);
-      hipLaunchKernelGGL(fwd::prefixlm_fwd_kernel<HD>, dim3((unsigned)(nblk + npad)), dim3(fwd::NT),
-                         fwd::Geo<HD>::LDS_BYTES, stream, P);
+      if (split)
+        hipLaunchKernelGGL((fwd::prefixlm_fwd_kernel<HD, false, 2>), dim3((unsigned)(nblk + npad)), dim3(nt),
+                           2 * fwd::Geo<HD>::LDS_BYTES, stream, P);
+      else
+        hipLaunchKernelGGL(fwd::prefixlm_fwd_kernel<HD>, dim3((unsigned)(nblk + npad)), dim3(nt),
+                           fwd::Geo<HD>::LDS_BYTES, stream, P);
     }
   }
   const hipError_t e = hipGetLastError();
@@ -1119,11 +1146,19 @@ int prefixlm_kvcache_fwd(const prefixlm_kvcache_args* a, void* stream_) {
     F.kc_sb = P.kc_sb; F.kc_ss = P.kc_ss; F.kc_sh = P.kc_sh;
     F.vc_sb = P.vc_sb; F.vc_ss = P.vc_ss; F.vc_sh = P.vc_sh;
     const int64_t items = (int64_t)B * ((S + fwd::BM - 1) / fwd::BM), nblk = unit_grid(items, H);
-    const int64_t nappend = (T * H * 16 + fwd::NT * fwd::kAppend - 1) / (fwd::NT * fwd::kAppend);
+    bool split = false;
+    const int rc2 = fwd_splits_keys(nblk, S, &split);
+    if (rc2) return rc2;
+    const int nt = fwd::NT * (split ? 2 : 1), per = nt * fwd::kAppend;
+    const int64_t nappend = (T * H * 16 + per - 1) / per;
     if (nblk + nappend > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "grid too large");
     F.n_main = (int)nblk;
-    hipLaunchKernelGGL((fwd::prefixlm_fwd_kernel<kvc::D, true>), dim3((unsigned)(nblk + nappend)), dim3(fwd::NT),
-                       fwd::Geo<kvc::D>::LDS_BYTES, stream, F);
+    if (split)
+      hipLaunchKernelGGL((fwd::prefixlm_fwd_kernel<kvc::D, true, 2>), dim3((unsigned)(nblk + nappend)), dim3(nt),
+                         2 * fwd::Geo<kvc::D>::LDS_BYTES, stream, F);
+    else
+      hipLaunchKernelGGL((fwd::prefixlm_fwd_kernel<kvc::D, true>), dim3((unsigned)(nblk + nappend)), dim3(nt),
+                         fwd::Geo<kvc::D>::LDS_BYTES, stream, F);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(PREFIXLM_ERR_HIP, "prefill launch: %s", hipGetErrorString(e));
     return PREFIXLM_OK;
