@@ -390,7 +390,7 @@ __global__ __launch_bounds__(64 * NWV, 1) void proj_skinny_kernel(Params P, floa
 #pragma unroll
       for (int v = 0; v < NWV; ++v) s += sums[(v * MB + m) * 32 + l32];
       rs = __builtin_amdgcn_rsqf(s / (float)P.K + eps);
-      if (blockIdx.x == 0 && w == 0 && hh == 0 && row < P.M) rstd_out[row] = rs;
+      if (rstd_out != nullptr && blockIdx.x == 0 && w == 0 && hh == 0 && row < P.M) rstd_out[row] = rs;
     }
     float t[NB][RW];
 #pragma unroll

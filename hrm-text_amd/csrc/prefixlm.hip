@@ -857,6 +857,15 @@ static void (*rmsnorm_kernel(int cols, bool backward))(nm::NormParams) {
   }
 }
 
+static void (*add_rmsnorm_kernel(int cols))(nm::NormParams) {
+  const int need = (cols / 8 + 63) / 64;
+  return need <= 1   ? nm::rmsnorm_fwd_kernel<1, true>
+         : need <= 2 ? nm::rmsnorm_fwd_kernel<2, true>
+         : need <= 4 ? nm::rmsnorm_fwd_kernel<4, true>
+         : need <= 8 ? nm::rmsnorm_fwd_kernel<8, true>
+                     : nm::rmsnorm_fwd_kernel<16, true>;
+}
+
 static int rmsnorm_launch(const prefixlm_rmsnorm_args* a, void* stream_, bool backward) {
   if (!a) return fail(PREFIXLM_ERR_INVALID, "args is null");
   if (a->rows < 0 || a->cols < 8 || a->cols % 8 || a->cols > nm::kNormMaxCols)
@@ -877,7 +886,7 @@ static int rmsnorm_launch(const prefixlm_rmsnorm_args* a, void* stream_, bool ba
   if ((a->rows + 3) / 4 > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "too many rows");
   nm::NormParams P{static_cast<const bf16*>(a->x), static_cast<const bf16*>(a->dy), static_cast<bf16*>(a->y),
                    static_cast<bf16*>(a->dx), a->rstd, a->x_stride, a->y_stride, a->dy_stride, a->dx_stride,
-                   a->rows, a->cols, a->eps};
+                   a->rows, a->cols, a->eps, nullptr, nullptr, 0, 0};
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
   (void)hipGetLastError();
   hipLaunchKernelGGL(rmsnorm_kernel(a->cols, backward), dim3((unsigned)((a->rows + 3) / 4)), dim3(256), 0, stream, P);
@@ -888,6 +897,34 @@ static int rmsnorm_launch(const prefixlm_rmsnorm_args* a, void* stream_, bool ba
 
 int prefixlm_rmsnorm_fwd(const prefixlm_rmsnorm_args* a, void* stream) { return rmsnorm_launch(a, stream, false); }
 int prefixlm_rmsnorm_bwd(const prefixlm_rmsnorm_args* a, void* stream) { return rmsnorm_launch(a, stream, true); }
+
+int prefixlm_add_rmsnorm(const prefixlm_add_rmsnorm_args* a, void* stream_) {
+  if (!a) return fail(PREFIXLM_ERR_INVALID, "args is null");
+  if (a->rows < 0 || a->cols < 8 || a->cols % 8 || a->cols > nm::kNormMaxCols)
+    return fail(PREFIXLM_ERR_INVALID, "rows=%lld cols=%d: cols must be a multiple of 8 in [8, %d]",
+                (long long)a->rows, a->cols, nm::kNormMaxCols);
+  if (!(a->eps >= 0.f)) return fail(PREFIXLM_ERR_INVALID, "eps must be >= 0");
+  if (a->rows == 0) return PREFIXLM_OK;   // empty tensors may have null pointers
+  const void* ptrs[] = {a->x, a->r, a->s, a->y};
+  const int64_t st[] = {a->x_stride, a->r_stride, a->s_stride, a->y_stride};
+  for (int i = 0; i < (a->y ? 4 : 3); ++i) {
+    if (!ptrs[i] || !aligned16(ptrs[i]))
+      return fail(PREFIXLM_ERR_INVALID, "pointer %d is null or not 16-byte aligned", i);
+    if ((st[i] < a->cols && !(i < 2 && st[i] == 0)) || st[i] % 8)
+      return fail(PREFIXLM_ERR_INVALID, "row stride %d (%lld) must be a multiple of 8 and >= cols", i, (long long)st[i]);
+  }
+  if (!a->rstd) return fail(PREFIXLM_ERR_INVALID, "rstd is null");
+  if ((a->rows + 3) / 4 > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "too many rows");
+  const nm::NormParams P{static_cast<const bf16*>(a->x), nullptr, static_cast<bf16*>(a->y), nullptr, a->rstd, a->x_stride,
+                         a->y_stride, 0, 0, a->rows, a->cols, a->eps, static_cast<const bf16*>(a->r),
+                         static_cast<bf16*>(a->s), a->r_stride, a->s_stride};
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(add_rmsnorm_kernel(a->cols), dim3((unsigned)((a->rows + 3) / 4)), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream_), P);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(PREFIXLM_ERR_HIP, "add + rmsnorm launch: %s", hipGetErrorString(e));
+  return PREFIXLM_OK;
+}
 
 }  // extern "C"
 
@@ -912,18 +949,20 @@ static int proj_skinny_launch(const mlp::Params& P, bool sw, bool norm, float* r
   if (e != hipSuccess) return fail(PREFIXLM_ERR_HIP, "projection launch: %s", hipGetErrorString(e));
   return PREFIXLM_OK;
 }
-static int proj_skinny(const prefixlm_proj_gemm_args* a, hipStream_t stream) {
+static int proj_skinny(const prefixlm_proj_gemm_args* a, bool given, hipStream_t stream) {
   const mlp::Params P{static_cast<const bf16*>(a->x), static_cast<const bf16*>(a->w), static_cast<bf16*>(a->y),
                       nullptr, a->x_stride, a->w_stride, a->y_stride, a->M, a->K, a->N, 0, 0};
   const bool sw = a->swiglu != 0, norm = a->norm != 0;
-  if (a->M <= 32) return proj_skinny_launch<1, 8>(P, sw, norm, a->rstd, a->eps, stream);
-  if (a->M <= 64) return proj_skinny_launch<2, 8>(P, sw, norm, a->rstd, a->eps, stream);
-  return proj_skinny_launch<4, 4>(P, sw, norm, a->rstd, a->eps, stream);
+  float* const rstd = given ? nullptr : a->rstd;   // given ones are found again from x
+  if (a->M <= 32) return proj_skinny_launch<1, 8>(P, sw, norm, rstd, a->eps, stream);
+  if (a->M <= 64) return proj_skinny_launch<2, 8>(P, sw, norm, rstd, a->eps, stream);
+  return proj_skinny_launch<4, 4>(P, sw, norm, rstd, a->eps, stream);
 }
 
 extern "C" {
 
-int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
+// given: the row scales are in a->rstd already
+static int proj_gemm_launch(const prefixlm_proj_gemm_args* a, void* stream_, bool given) {
   if (!a) return fail(PREFIXLM_ERR_INVALID, "args is null");
   const bool sw = a->swiglu != 0;
   if (a->M < 0 || a->K < mlp::KT || a->K % mlp::KT || a->N < mlp::WT || a->N % mlp::WT)
@@ -939,6 +978,7 @@ int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
     return fail(PREFIXLM_ERR_INVALID, "strides (x %lld, w %lld, y %lld) must be multiples of 8 covering the rows",
                 (long long)a->x_stride, (long long)a->w_stride, (long long)a->y_stride);
   if (!(a->eps >= 0.f)) return fail(PREFIXLM_ERR_INVALID, "eps must be >= 0");
+  if (given && !a->norm) return fail(PREFIXLM_ERR_INVALID, "row scales without norm");
   if (a->norm) {
     if (!a->rstd) return fail(PREFIXLM_ERR_INVALID, "norm needs rstd (M floats)");
     if (a->K > nm::kNormMaxCols) return fail(PREFIXLM_ERR_INVALID, "norm: K=%d exceeds %d", a->K, nm::kNormMaxCols);
@@ -949,7 +989,7 @@ int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
     return fail(PREFIXLM_ERR_INVALID, "operands exceed the 32-bit offsets of the kernel");
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
   (void)hipGetLastError();
-  if (a->M <= 128) return proj_skinny(a, stream);
+  if (a->M <= 128) return proj_skinny(a, given, stream);
   int cus = 0;
   const int rc = persistent_grid(&cus);
   if (rc) return rc;
@@ -979,10 +1019,10 @@ int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
                                      i < 4 ? mlp::Geo<256>::LDS_BYTES : mlp::Geo<128>::LDS_BYTES);
   });
   if (attr_err != hipSuccess) return fail(PREFIXLM_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
-  if (a->norm) {
+  if (a->norm && !given) {
     // the row scales first (a wave per row, x read once; the normalized x is not written)
     nm::NormParams N{static_cast<const bf16*>(a->x), nullptr, nullptr, nullptr, a->rstd, a->x_stride, 0, 0, 0,
-                     a->M, a->K, a->eps};
+                     a->M, a->K, a->eps, nullptr, nullptr, 0, 0};
     hipLaunchKernelGGL(rmsnorm_kernel(a->K, false), dim3((unsigned)((a->M + 3) / 4)), dim3(256), 0, stream, N);
   }
   hipLaunchKernelGGL(kernels[4 * (half ? 1 : 0) + 2 * (sw ? 1 : 0) + (a->norm ? 1 : 0)], dim3(grid), dim3(mlp::NTH),
@@ -990,6 +1030,12 @@ int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream_) {
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(PREFIXLM_ERR_HIP, "projection gemm launch: %s", hipGetErrorString(e));
   return PREFIXLM_OK;
+}
+
+int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* a, void* stream) { return proj_gemm_launch(a, stream, false); }
+
+int prefixlm_proj_gemm_scaled(const prefixlm_proj_gemm_args* a, void* stream) {
+  return proj_gemm_launch(a, stream, true);
 }
 
 // Whether the 256-byte rows of a [B, N, H] cache with these element strides are all apart:

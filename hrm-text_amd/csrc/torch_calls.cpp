@@ -56,7 +56,9 @@ struct Lib {
   decltype(&prefixlm_swiglu_bwd) swiglu_bwd;
   decltype(&prefixlm_rmsnorm_fwd) rmsnorm_fwd;
   decltype(&prefixlm_rmsnorm_bwd) rmsnorm_bwd;
+  decltype(&prefixlm_add_rmsnorm) add_rmsnorm;
   decltype(&prefixlm_proj_gemm) proj_gemm;
+  decltype(&prefixlm_proj_gemm_scaled) proj_gemm_scaled;
   decltype(&prefixlm_kvcache_workspace_size) kv_ws;
   decltype(&prefixlm_kvcache_fwd) kv_fwd;
   decltype(&prefixlm_last_error) last_error;
@@ -465,8 +467,8 @@ struct Layer : torch::autograd::Function<Layer> {
 };
 
 // ---- the block's norm and activation ----------------------------------------------------------
-// x as [rows, cols] with 16-byte rows, or undefined
-Tensor rows_view(const Tensor& x) {
+// x as [rows, cols] with 16-byte rows, or undefined; one row repeated only with `repeated`
+Tensor rows_view(const Tensor& x, bool repeated = false) {
   if (x.scalar_type() != at::kBFloat16 || x.dim() < 1 || x.size(-1) < 1 || x.numel() == 0) return Tensor();
   Tensor r;
   if (x.dim() == 2) {
@@ -475,7 +477,10 @@ Tensor rows_view(const Tensor& x) {
     if (!x.is_contiguous()) return Tensor();
     r = x.view({-1, x.size(-1)});
   }
-  return r.stride(1) == 1 && r.stride(0) % 8 == 0 && r.stride(0) >= r.size(1) && aligned(r, 16) ? r : Tensor();
+  return r.stride(1) == 1 && r.stride(0) % 8 == 0 &&
+                 (r.stride(0) >= r.size(1) || (repeated && r.stride(0) == 0)) && aligned(r, 16)
+             ? r
+             : Tensor();
 }
 Tensor rows_of(const Tensor& x) {   // a gradient: copied where its layout does not serve
   const Tensor r = rows_view(x);
@@ -744,6 +749,87 @@ PyObject* py_rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// x, r, eps, with_y -> (x + r, its norm) or (x + r, its row scales)
+PyObject* py_add_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Tensor x, r;
+  double eps;
+  bool with_y;
+  if (!ready(n, 4) || c10::InferenceMode::is_enabled()) return none();
+  if (!get_tensor(a[0], &x) || !get_tensor(a[1], &r) || !get_double(a[2], &eps) || !get_bool(a[3], &with_y) ||
+      wants_grad(x) || wants_grad(r) || x.sizes() != r.sizes() || x.device() != r.device())
+    return none();
+  Tensor s, y;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const at::NoGradGuard no_grad;
+    const Tensor x2 = rows_view(x, true), r2 = rows_view(r, true);
+    if (x2.defined() && r2.defined() && x2.size(1) <= INT32_MAX) {
+      const c10::DeviceGuard guard(x.device());
+      s = empty_like_on(x, x.sizes(), at::kBFloat16);
+      if (with_y) y = empty_like_on(x, x.sizes(), at::kBFloat16);
+      const Tensor rstd = empty_like_on(x, {x2.size(0)}, at::kFloat);
+      prefixlm_add_rmsnorm_args p{};
+      p.x = x2.const_data_ptr();
+      p.r = r2.const_data_ptr();
+      p.s = s.data_ptr();
+      p.y = with_y ? y.data_ptr() : nullptr;
+      p.rstd = rstd.data_ptr<float>();
+      p.x_stride = x2.stride(0);
+      p.r_stride = r2.stride(0);
+      p.s_stride = p.y_stride = x2.size(1);
+      p.rows = x2.size(0);
+      p.cols = (int32_t)x2.size(1);
+      p.eps = (float)eps;
+      check(lib.add_rmsnorm(&p, stream_of(x)), "prefixlm_add_rmsnorm");
+      if (!with_y) y = rstd;
+    }
+  }
+  if (!s.defined()) return none();
+  PyObject* t = PyTuple_New(2);
+  if (!t) return nullptr;
+  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(s));
+  PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(y));
+  return t;
+  END_HANDLE_TH_ERRORS
+}
+
+// The projection of x by w; scales: the row scales of x, or undefined (norm says whether the
+// call finds them itself). Undefined for operands that are not plain.
+Tensor projection(const Tensor& x, const Tensor& w, const Tensor& scales, bool sw, bool norm, double eps) {
+  const at::NoGradGuard no_grad;
+  const Tensor x2 = rows_view(x);
+  if (!x2.defined() || w.scalar_type() != at::kBFloat16 || w.dim() != 2 || w.device() != x.device() ||
+      w.stride(1) != 1 || w.stride(0) % 8 || !aligned(w, 16) || w.size(1) != x2.size(1) || x2.size(0) > INT32_MAX ||
+      w.size(0) > INT32_MAX)
+    return Tensor();
+  const c10::DeviceGuard guard(x.device());
+  const int64_t M = x2.size(0), N = w.size(0), nout = sw ? N / 2 : N;
+  auto sizes = x.sizes().vec();
+  sizes.back() = nout;
+  const Tensor y = empty_like_on(x, sizes, at::kBFloat16);
+  Tensor rstd = scales;
+  prefixlm_proj_gemm_args p{};
+  if (norm && !rstd.defined()) rstd = empty_like_on(x, {M}, at::kFloat);
+  if (rstd.defined()) p.rstd = rstd.data_ptr<float>();
+  p.x = x2.const_data_ptr();
+  p.w = w.const_data_ptr();
+  p.y = y.data_ptr();
+  p.x_stride = x2.stride(0);
+  p.w_stride = w.stride(0);
+  p.y_stride = nout;
+  p.M = (int32_t)M;
+  p.K = (int32_t)x2.size(1);
+  p.N = (int32_t)N;
+  p.swiglu = i32(sw);
+  p.norm = i32(norm);
+  p.eps = (float)eps;
+  if (scales.defined())
+    check(lib.proj_gemm_scaled(&p, stream_of(x)), "prefixlm_proj_gemm_scaled");
+  else
+    check(lib.proj_gemm(&p, stream_of(x)), "prefixlm_proj_gemm");
+  return y;
+}
 // x, w, swiglu, norm, eps
 PyObject* py_proj_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -757,36 +843,28 @@ PyObject* py_proj_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor y;
   {
     pybind11::gil_scoped_release no_gil;
-    const at::NoGradGuard no_grad;
-    const Tensor x2 = rows_view(x);
-    if (x2.defined() && w.scalar_type() == at::kBFloat16 && w.dim() == 2 && w.device() == x.device() &&
-        w.stride(1) == 1 && w.stride(0) % 8 == 0 && aligned(w, 16) && w.size(1) == x2.size(1) &&
-        x2.size(0) <= INT32_MAX && w.size(0) <= INT32_MAX) {
-      const c10::DeviceGuard guard(x.device());
-      const int64_t M = x2.size(0), N = w.size(0), nout = sw ? N / 2 : N;
-      auto sizes = x.sizes().vec();
-      sizes.back() = nout;
-      y = empty_like_on(x, sizes, at::kBFloat16);
-      Tensor rstd;
-      prefixlm_proj_gemm_args p{};
-      if (norm) {
-        rstd = empty_like_on(x, {M}, at::kFloat);
-        p.rstd = rstd.data_ptr<float>();
-      }
-      p.x = x2.const_data_ptr();
-      p.w = w.const_data_ptr();
-      p.y = y.data_ptr();
-      p.x_stride = x2.stride(0);
-      p.w_stride = w.stride(0);
-      p.y_stride = nout;
-      p.M = (int32_t)M;
-      p.K = (int32_t)x2.size(1);
-      p.N = (int32_t)N;
-      p.swiglu = i32(sw);
-      p.norm = i32(norm);
-      p.eps = (float)eps;
-      check(lib.proj_gemm(&p, stream_of(x)), "prefixlm_proj_gemm");
-    }
+    y = projection(x, w, Tensor(), sw, norm, eps);
+  }
+  return y.defined() ? THPVariable_Wrap(y) : none();
+  END_HANDLE_TH_ERRORS
+}
+// x, w, rstd, swiglu, eps
+PyObject* py_proj_gemm_scaled(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Tensor x, w, rstd;
+  bool sw;
+  double eps;
+  if (!ready(n, 5) || c10::InferenceMode::is_enabled()) return none();
+  if (!get_tensor(a[0], &x) || !get_tensor(a[1], &w) || !get_tensor(a[2], &rstd) || !get_bool(a[3], &sw) ||
+      !get_double(a[4], &eps) || wants_grad(x) || wants_grad(w) || wants_grad(rstd))
+    return none();
+  if (rstd.scalar_type() != at::kFloat || rstd.device() != x.device() || !rstd.is_contiguous() || x.dim() < 1 ||
+      x.size(-1) < 1 || rstd.numel() != x.numel() / x.size(-1))
+    return none();
+  Tensor y;
+  {
+    pybind11::gil_scoped_release no_gil;
+    y = projection(x, w, rstd, sw, true, eps);
   }
   return y.defined() ? THPVariable_Wrap(y) : none();
   END_HANDLE_TH_ERRORS
@@ -822,7 +900,9 @@ PyMethodDef methods[] = {
     {"kvcache", FAST(py_kvcache), nullptr},
     {"swiglu", FAST(py_swiglu), nullptr},
     {"rms_norm", FAST(py_rms_norm), nullptr},
+    {"add_rmsnorm", FAST(py_add_rmsnorm), nullptr},
     {"proj_gemm", FAST(py_proj_gemm), nullptr},
+    {"proj_gemm_scaled", FAST(py_proj_gemm_scaled), nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -128,6 +128,14 @@ class RmsnormArgs(ctypes.Structure):
     ]
 
 
+class AddRmsnormArgs(ctypes.Structure):
+    _fields_ = [
+        ("x", c_vp), ("r", c_vp), ("s", c_vp), ("y", c_vp), ("rstd", c_vp),
+        ("x_stride", c_i64), ("r_stride", c_i64), ("s_stride", c_i64), ("y_stride", c_i64),
+        ("rows", c_i64), ("cols", c_i32), ("eps", c_f32),
+    ]
+
+
 class ProjGemmArgs(ctypes.Structure):
     _fields_ = [
         ("x", c_vp), ("w", c_vp), ("y", c_vp),
@@ -156,6 +164,8 @@ SIGNATURES = {
     "prefixlm_swiglu_bwd": (ctypes.c_int, [ctypes.POINTER(SwigluArgs), c_vp]),
     "prefixlm_rmsnorm_fwd": (ctypes.c_int, [ctypes.POINTER(RmsnormArgs), c_vp]),
     "prefixlm_rmsnorm_bwd": (ctypes.c_int, [ctypes.POINTER(RmsnormArgs), c_vp]),
+    "prefixlm_add_rmsnorm": (ctypes.c_int, [ctypes.POINTER(AddRmsnormArgs), c_vp]),
+    "prefixlm_proj_gemm_scaled": (ctypes.c_int, [ctypes.POINTER(ProjGemmArgs), c_vp]),
     "prefixlm_proj_gemm": (ctypes.c_int, [ctypes.POINTER(ProjGemmArgs), c_vp]),
     "prefixlm_kvcache_workspace_size": (c_sz, [c_i32, c_i32, c_i32, c_i32, c_i32]),
     "prefixlm_kvcache_fwd": (ctypes.c_int, [ctypes.POINTER(KvcacheArgs), c_vp]),

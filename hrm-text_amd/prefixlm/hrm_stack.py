@@ -33,8 +33,10 @@ from dataclasses import dataclass
 from typing import Callable, Optional
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 from torch import Tensor, nn
+from torch.nn.modules.module import _has_any_global_hook
 
 __all__ = ["HRMStackConfig", "HRMStack", "FusedLayer", "rotary_cos_sin", "apply_rotary", "intermediate_size"]
 
@@ -155,7 +157,11 @@ class _SwiGLU(nn.Module):
         self.gate_up = nn.Parameter(torch.empty(2 * cfg.ffn, cfg.hidden_size))
         self.down = nn.Parameter(torch.empty(cfg.hidden_size, cfg.ffn))
 
-    def forward(self, x: Tensor, prenormed: bool = True) -> Tensor:
+    def forward(self, x: Tensor, prenormed: bool = True, rstd: Optional[Tensor] = None) -> Tensor:
+        if rstd is not None:
+            # x still needs its norm, whose row scales are rstd
+            from .norm_mlp import rms_scaled_swiglu
+            return F.linear(rms_scaled_swiglu(x, self.gate_up, rstd, self.cfg.norm_eps), self.down)
         if not prenormed:
             # pre-norm, gate_up projection and SwiGLU in one GEMM
             from .norm_mlp import rms_norm_swiglu
@@ -185,6 +191,11 @@ class _Block(nn.Module):
         return x + self.mlp(self.norm(x))
 
 
+def _called_plainly(m: nn.Module, cls) -> bool:
+    return (type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks
+            and "forward" not in m.__dict__ and m._compiled_call_impl is None)
+
+
 class _Module(nn.Module):
     """One recurrent module (H or L): input injection, layers, final norm."""
 
@@ -193,7 +204,41 @@ class _Module(nn.Module):
         self.cfg = cfg
         self.layers = nn.ModuleList(_Block(cfg) for _ in range(cfg.layers_per_module))
 
+    def _adds_fuse(self, hidden, injection) -> bool:
+        """Whether the residual adds can run inside the norms' kernel: an eager call without
+        gradients of either mode through the HIP elementwise kernels, over blocks that are called
+        as they stand (no hook or replaced forward that wants a block's own input and output)."""
+        if not (self.cfg.fused_elementwise and not torch.is_grad_enabled() and not torch.compiler.is_compiling()):
+            return False
+        for t in (hidden, injection):
+            if type(t) is not Tensor or t.device.type != "cuda" or t.dtype != torch.bfloat16 \
+                    or fwAD.unpack_dual(t).tangent is not None:
+                return False
+        return (hidden.shape == injection.shape and hidden.device == injection.device and not _has_any_global_hook()
+                and all(_called_plainly(b, _Block) and _called_plainly(b.mlp, _SwiGLU) for b in self.layers))
+
+    def _forward_fused_adds(self, hidden, injection, cos, sin, attn, seq_info):
+        """The blocks with each residual add and the norm after it as one kernel (bitwise the
+        separate ones)."""
+        from .norm_mlp import add_rms_norm, add_rms_scales
+        eps = self.cfg.norm_eps
+        x, n = add_rms_norm(hidden, injection, eps)
+        for b in self.layers:
+            a = b.attn(n, cos, sin, attn, seq_info)
+            del n
+            if self.cfg.fused_gemm:
+                x, rstd = add_rms_scales(x, a, eps)
+                m = b.mlp(x, rstd=rstd)
+            else:
+                x, n = add_rms_norm(x, a, eps)
+                m = b.mlp(n)
+            x, n = add_rms_norm(x, m, eps)
+            del a, m
+        return n
+
     def forward(self, hidden, injection, cos, sin, attn, seq_info):
+        if self._adds_fuse(hidden, injection):
+            return self._forward_fused_adds(hidden, injection, cos, sin, attn, seq_info)
         x = hidden + injection
         for layer in self.layers:
             x = layer(x, cos, sin, attn, seq_info)

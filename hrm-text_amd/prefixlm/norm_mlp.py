@@ -160,6 +160,51 @@ def rms_norm(x: Tensor, eps: float = 1e-6) -> Tensor:
     return RMSNormFunction.apply(x, eps) if y is None else y
 
 
+# ---- the residual add with the norm after it (forward only) ------------------------------
+@torch.library.custom_op("prefixlm::add_rmsnorm", mutates_args=())
+def add_rmsnorm(x: Tensor, r: Tensor, eps: float, with_y: bool) -> Tuple[Tensor, Tensor, Tensor]:
+    """(s, y, rstd): s = x + r in bf16, rstd fp32 [rows] of s and y = s * rstd (empty without
+    ``with_y``). Forward only: the op has no autograd formula."""
+    if tuple(x.shape) != tuple(r.shape) or r.device != x.device:
+        raise ValueError(f"x {tuple(x.shape)} on {x.device} and r {tuple(r.shape)} on {r.device} do not match")
+    lib = _capi.load()
+    # one repeated row (stride 0) is read in place; rows that overlap otherwise and contiguous
+    # ones off their 16 bytes are copied
+    x2, r2 = (t.clone(memory_format=torch.contiguous_format)
+              if t.data_ptr() % 16 or 0 < t.stride(0) < t.shape[1] else t for t in (_rows(x, "x"), _rows(r, "r")))
+    rows, cols = x2.shape
+    s = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    y = torch.empty(x.shape if with_y else (0,), dtype=x.dtype, device=x.device)
+    rstd = torch.empty(rows, dtype=torch.float32, device=x.device)
+    a = _capi.AddRmsnormArgs(_ptr(x2), _ptr(r2), _ptr(s), _ptr(y) if with_y else None, _ptr(rstd), x2.stride(0),
+                             r2.stride(0), cols, cols, rows, cols, float(eps))
+    with torch.cuda.device(x.device):
+        _capi.check(lib.prefixlm_add_rmsnorm(ctypes.byref(a), _stream(x.device)), "prefixlm_add_rmsnorm")
+    return s, y, rstd
+
+
+@add_rmsnorm.register_fake
+def _add_rmsnorm_fake(x, r, eps, with_y):
+    rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
+    return (x.new_empty(x.shape), x.new_empty(x.shape if with_y else (0,)),
+            x.new_empty((rows,), dtype=torch.float32))
+
+
+def add_rms_norm(x: Tensor, r: Tensor, eps: float) -> Tuple[Tensor, Tensor]:
+    """(s, y): ``s = x + r`` and ``y = rms_norm(s, eps)``, bitwise, in one pass (forward only)."""
+    native = _native_calls()
+    out = native.add_rmsnorm(x, r, eps, True) if native is not None else None
+    return add_rmsnorm(x, r, eps, True)[:2] if out is None else out
+
+
+def add_rms_scales(x: Tensor, r: Tensor, eps: float) -> Tuple[Tensor, Tensor]:
+    """(s, rstd): ``s = x + r`` and the fp32 row scales that ``rms_norm(s, eps)`` applies, for
+    ``rms_scaled_swiglu`` (forward only)."""
+    native = _native_calls()
+    out = native.add_rmsnorm(x, r, eps, False) if native is not None else None
+    return add_rmsnorm(x, r, eps, False)[::2] if out is None else out
+
+
 # ---- projections with the norm and the SwiGLU fused in (forward only) ------------------
 @torch.library.custom_op("prefixlm::proj_gemm", mutates_args=())
 def proj_gemm(x: Tensor, w: Tensor, swiglu: bool, norm: bool, eps: float) -> Tensor:
@@ -183,6 +228,36 @@ def proj_gemm(x: Tensor, w: Tensor, swiglu: bool, norm: bool, eps: float) -> Ten
     with torch.cuda.device(x.device):
         _capi.check(lib.prefixlm_proj_gemm(ctypes.byref(a), _stream(x.device)), "prefixlm_proj_gemm")
     return y.view(*x.shape[:-1], nout)
+
+
+@torch.library.custom_op("prefixlm::proj_gemm_scaled", mutates_args=())
+def proj_gemm_scaled(x: Tensor, w: Tensor, rstd: Tensor, swiglu: bool, eps: float) -> Tensor:
+    """proj_gemm with the norm, its row scales given (those of x at ``eps``, from
+    ``add_rms_scales``): no row pass over x."""
+    lib = _capi.load()
+    x2 = _rows(x, "x")
+    if w.dtype != torch.bfloat16 or w.dim() != 2 or w.device != x.device:
+        raise ValueError(f"w must be a bf16 [N, K] tensor on {x.device}")
+    w2 = w if (w.stride(-1) == 1 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0) else w.contiguous()
+    M, K = x2.shape
+    N = w2.shape[0]
+    if w2.shape[1] != K:
+        raise ValueError(f"w is [{N}, {w2.shape[1]}], x has K = {K}")
+    if rstd.dtype != torch.float32 or rstd.numel() != M or rstd.device != x.device:
+        raise ValueError(f"rstd must be float32 [{M}] (got {rstd.dtype} {tuple(rstd.shape)})")
+    rstd = rstd.contiguous()
+    nout = N // 2 if swiglu else N
+    y = torch.empty((M, nout), dtype=x.dtype, device=x.device)
+    a = _capi.ProjGemmArgs(_ptr(x2), _ptr(w2), _ptr(y), x2.stride(0), w2.stride(0), y.stride(0), M, K, N,
+                           1 if swiglu else 0, 1, float(eps), _ptr(rstd))
+    with torch.cuda.device(x.device):
+        _capi.check(lib.prefixlm_proj_gemm_scaled(ctypes.byref(a), _stream(x.device)), "prefixlm_proj_gemm_scaled")
+    return y.view(*x.shape[:-1], nout)
+
+
+@proj_gemm_scaled.register_fake
+def _proj_gemm_scaled_fake(x, w, rstd, swiglu, eps):
+    return x.new_empty((*x.shape[:-1], w.shape[0] // 2 if swiglu else w.shape[0]))
 
 
 @proj_gemm.register_fake
@@ -215,3 +290,10 @@ def rms_norm_swiglu(x: Tensor, w_gate_up: Tensor, eps: float) -> Tensor:
     slower than hipBLASLt's (about 1.22 vs 1.44 PFLOP/s), which cancels the saving inside
     the config-5 stack (150.5 vs 149.6 ms per step with and without it)."""
     return _proj(x, w_gate_up, True, float(eps))
+
+
+def rms_scaled_swiglu(x: Tensor, w_gate_up: Tensor, rstd: Tensor, eps: float) -> Tensor:
+    """``rms_norm_swiglu`` with the row scales of x given (``add_rms_scales``)."""
+    native = _native_calls()
+    y = native.proj_gemm_scaled(x, w_gate_up, rstd, True, eps) if native is not None else None
+    return proj_gemm_scaled(x, w_gate_up, rstd, True, eps) if y is None else y

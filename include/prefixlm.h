@@ -282,6 +282,23 @@ typedef struct prefixlm_rmsnorm_args {
 int prefixlm_rmsnorm_fwd(const prefixlm_rmsnorm_args* args, void* stream);
 int prefixlm_rmsnorm_bwd(const prefixlm_rmsnorm_args* args, void* stream);
 
+/* A residual add and the RMSNorm after it, x + attn(...) then norm (models/transformer.py:90-92),
+ * as one pass: s = bf16(x + r), rstd of the rows of s, and unless y is NULL y = s * rstd, each
+ * rounded as the separate operations round. Layouts as prefixlm_rmsnorm_fwd; x and r may repeat
+ * one row (row stride 0). Forward only. */
+typedef struct prefixlm_add_rmsnorm_args {
+  const void* x;
+  const void* r;
+  void* s;
+  void* y;                       /* optional (NULL: only s and rstd) */
+  float* rstd;                   /* fp32 [rows] */
+  int64_t x_stride, r_stride, s_stride, y_stride;
+  int64_t rows;
+  int32_t cols;
+  float eps;
+} prefixlm_add_rmsnorm_args;
+int prefixlm_add_rmsnorm(const prefixlm_add_rmsnorm_args* args, void* stream);
+
 /* Projection GEMM of the block with the pre-norm RMSNorm fused in, and optionally the MLP's
  * SwiGLU (models/transformer.py:87-92, models/layers.py:124-135, :158-168):
  *   swiglu = 0: y = rmsnorm(x) W^T                         (y: [M, N])
@@ -307,6 +324,9 @@ typedef struct prefixlm_proj_gemm_args {
   float* rstd;                   /* [M] fp32, written when norm != 0 */
 } prefixlm_proj_gemm_args;
 int prefixlm_proj_gemm(const prefixlm_proj_gemm_args* args, void* stream);
+/* The same product with norm = 1 whose row scales are given: rstd is read, not written (those of
+ * x at eps, from prefixlm_add_rmsnorm), and the pass over x that finds them is left out. */
+int prefixlm_proj_gemm_scaled(const prefixlm_proj_gemm_args* args, void* stream);
 
 /* KV-cache attention, the inference path of the reference's attention layer
  * (flash_attn_with_kvcache, models/layers.py:147-151, simple_inference_engine.py:105-112).
