@@ -202,6 +202,20 @@ int fwd_splits_keys(int64_t grid, int32_t max_all, bool* split) {
   return rc;
 }
 
+// Whether the forward's workgroups find their items themselves instead of reading a cost-ordered
+// list, which a launch before it would have to build (about 4.8 us). The order only matters once
+// workgroups wait for others: grids of up to 1.25 workgroups per CU gain the whole launch (H 16 x
+// d128, us with and without the list: 2048 rows in 4 segments, 320 workgroups, 33.2 and 28.1; 280
+// 53.9 and 49.0; but 536 with segments of up to 4096 rows 128 and 142), and where no segment is
+// longer than 1024 rows, grids of up to three per CU (416 workgroups 21.3 and 16.2, 640 39.5 and
+// 36.7; at 1280 56.1 and 56.4). One wave reads the metadata: 64 segments.
+int fwd_finds_items(int64_t grid, int32_t numseqs, int32_t max_all, bool* self) {
+  int cus = 0;
+  const int rc = persistent_grid(&cus);
+  *self = grid > 0 && numseqs <= 64 && (4 * grid <= 5 * (int64_t)cus || (max_all <= 1024 && grid <= 3 * (int64_t)cus));
+  return rc;
+}
+
 // Checks shared by forward and backward. `strides` lists (stride_t, stride_h) pairs.
 int check_common(const void* const* ptrs, int nptr, const int64_t* strides, int nstr,
                  int32_t T, int32_t H, int32_t D, int32_t total, int32_t numseqs,
@@ -373,8 +387,14 @@ static int fwd_launch(const prefixlm_fwd_args* a, void* stream_) {
   const int T = a->num_tokens, H = a->num_heads;
 
   (void)hipGetLastError();
+  const int64_t nblk = unit_grid(nmax, H);
+  bool self = false;
   if (!use_plan) {
-    // always run, so the workspace header (item count, error word) is fresh
+    rc = fwd_finds_items(nblk, a->numseqs, a->max_seqlen_all, &self);
+    if (rc) return rc;
+  }
+  if (!use_plan && !self) {
+    // one of the two always runs, so the workspace header (item count, error word) is fresh
     MetaParams m{a->prefix_lens, a->causal_lens, a->cu_seqlens, a->numseqs, a->total_seqlen, T,
                  a->is_causal ? 1 : 0, a->max_seqlen_all};
     KernelTimer tm(a->timer, 0, stream);
@@ -403,15 +423,16 @@ static int fwd_launch(const prefixlm_fwd_args* a, void* stream_) {
     P.prefix = a->prefix_lens;
     P.causal = a->causal_lens;
     P.cu = a->cu_seqlens;
-    P.items = items;
+    P.items = self ? nullptr : items;
     P.hdr = hdr;
     P.q_amax = a->q_amax;
+    P.max_items = (int)nmax;
+    P.max_all = a->max_seqlen_all;
     P.T = T;
     P.H = H;
     P.is_causal = a->is_causal ? 1 : 0;
     P.numseqs = a->numseqs;
     P.scale_log2 = a->softmax_scale * kLog2e;
-    const int64_t nblk = unit_grid(nmax, H);
     bool split = false;
     rc = fwd_splits_keys(nblk, a->max_seqlen_all, &split);
     if (rc) return rc;

@@ -202,8 +202,8 @@ def _check_plan_before_launch(plan: Optional[Tensor], meta, ds_blocks: int = 0):
 
 
 def _check_lists_after_launch(lib, ws: Optional[Tensor], device, plan=None):
-    """Checking mode: device-built work lists carry an error word the list kernel
-    wrote; reading it synchronizes with the stream."""
+    """Checking mode: without a plan the workspace carries an error word that the list
+    kernel, or a forward that needs no list, wrote; reading it synchronizes with the stream."""
     if _CHECK_METADATA and plan is None:
         err = ctypes.c_int32(0)
         _capi.check(lib.prefixlm_check_workspace(_ptr(ws), _stream(device), ctypes.byref(err)),
