@@ -1084,7 +1084,11 @@ static int64_t kv_nsplit(int64_t B, int S, int64_t H, int64_t Smax) {
     // and two splits each of 512 keys or more, which even out ragged lengths (1024 pairs x
     // 4096: 272 us at one split, 263 at two, 266 at four; 2048 pairs x 256: 41 at one, 46 at
     // two).
+    // Caches of up to 256 rows: one split, whose keys take less time than the combine's launch
+    // (16 pairs x 128 keys 4.3 us, 6.9 with two splits; x 256 6.9 and 7.1 with four; x 384 9.3
+    // and 7.2).
     const int64_t units = B * H;
+    if (units <= 128 && Smax <= 256) return 1;
     if (units <= 128)
       return std::max<int64_t>(1, std::min({(512 + units - 1) / units, (Smax + kvc::kStep - 1) / kvc::kStep,
                                             (int64_t)kvc::kMaxSplits}));
@@ -1095,7 +1099,18 @@ static int64_t kv_nsplit(int64_t B, int S, int64_t H, int64_t Smax) {
   // merge: 4 x 16 heads x 45 queries 38 us a call at 512, 42 at 1024, 60 at 2048, and 2 x 16 x
   // 300 on 8192 rows 97 us at 512 against 103 at 256
   const int64_t want = (512 + units - 1) / units, most = (Smax + tk - 1) / tk;
-  return std::max<int64_t>(1, std::min({want, most, (int64_t)kvc::kMaxSplits}));
+  const int64_t n = std::max<int64_t>(1, std::min({want, most, (int64_t)kvc::kMaxSplits}));
+  // One split instead where the tiles it walks more cost less than the combine's launch and the
+  // partials, which n splits write and read for every query. Measured: a tile of 32, 64 or 128
+  // keys takes 1.27, 1.5 or 2.1 us with up to 512 workgroups, the launch 2.1 us at the least,
+  // a partial 0.2 ns. 256 pairs x 64 queries, one split against two: 128-row caches 15.4 and
+  // 32.0 us, 512 28.7 and 39.8, 1024 39.6 and 46.7; 64 pairs x 128 queries on 256 rows 24.1, and
+  // 28.3 with eight; 8 pairs x 64 queries on 256 rows 16.5, and 12.9 with the four it keeps.
+  const double c = ext_qw(S) == 1 ? 2100 : ext_qw(S) == 2 ? 1500 : 1270;   // ns
+  const double one = (double)most * c * std::max(1.0, (double)units / 512);
+  const double split = (double)((most + n - 1) / n) * c * std::max(1.0, (double)units * (double)n / 512) + 2100 +
+                       0.2 * (double)B * S * (double)H * (double)n;
+  return one <= split ? 1 : n;
 }
 
 size_t prefixlm_kvcache_workspace_size(int32_t batch, int32_t seqlen_q, int32_t num_heads, int32_t head_dim,
