@@ -24,8 +24,8 @@ __all__ = ["calls"]
 _ENTRY_POINTS = ("prefixlm_fwd", "prefixlm_bwd", "prefixlm_fwd_q_amax_count", "prefixlm_fwd_workspace_size",
                  "prefixlm_bwd_workspace_size", "prefixlm_bwd_ds_bytes", "prefixlm_bwd_ds_bytes_blocks",
                  "prefixlm_rope", "prefixlm_swiglu_fwd", "prefixlm_swiglu_bwd", "prefixlm_rmsnorm_fwd",
-                 "prefixlm_rmsnorm_bwd", "prefixlm_add_rmsnorm", "prefixlm_proj_gemm", "prefixlm_proj_gemm_scaled", "prefixlm_kvcache_workspace_size",
-                 "prefixlm_kvcache_fwd", "prefixlm_last_error")
+                 "prefixlm_rmsnorm_bwd", "prefixlm_add_rmsnorm", "prefixlm_proj_gemm", "prefixlm_proj_gemm_scaled",
+                 "prefixlm_kvcache_workspace_size", "prefixlm_kvcache_fwd", "prefixlm_last_error")
 
 _lock = threading.Lock()
 _module = None

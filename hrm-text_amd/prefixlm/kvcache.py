@@ -14,8 +14,9 @@ reference's engine drives it (simple_inference_engine.py:105-112, :179-180):
   and does not change results between calls (no atomics).
 
 A call with ``cache_seqlens`` the int 0 (the reference's prefill) runs the
-training forward kernels over the new rows; every other call runs a split-K
-decode kernel that reads each cached key and value once. The op is a
+training forward kernel over the new rows; every other call runs a split-K kernel:
+one query per row (decode) reads each cached key and value once, several queries
+share each read on the matrix cores. The op is a
 ``torch.library`` custom op mutating the caches, so ``torch.compile(fullgraph=True)``
 traces it (simple_inference_engine.py:105, :110).
 """

@@ -275,10 +275,9 @@ def _proj(x: Tensor, w: Tensor, swiglu: bool, eps: float) -> Tensor:
 def rms_norm_linear(x: Tensor, w: Tensor, eps: float) -> Tensor:
     """F.linear(F.rms_norm(x, (K,), eps), w) in one GEMM (forward only).
 
-    Not recommended for speed: the hand-written GEMM core runs at about 1.22 PFLOP/s on
-    the config-5 shapes against 1.44 for hipBLASLt, so at 2048 -> 8192 columns the norm
-    kernel plus the library GEMM is faster (0.38 vs 0.48 ms). Kept for callers that
-    want the normalized activations never written."""
+    Faster than the norm kernel plus the library's GEMM for few rows, slower for many: at
+    2048 -> 8192 columns 8.9 against 24.3 us for 16 rows, 23.1 and 24.9 for 128, 33.8 and
+    26.4 for 512, 493 and 414 for 16384. The normalized activations are never written."""
     return _proj(x, w, False, float(eps))
 
 
@@ -286,9 +285,10 @@ def rms_norm_swiglu(x: Tensor, w_gate_up: Tensor, eps: float) -> Tensor:
     """silu(g) * u for [g | u] = F.linear(F.rms_norm(x, (K,), eps), w_gate_up), in one
     GEMM (forward only).
 
-    Not recommended for speed: it saves the two elementwise passes but its GEMM core is
-    slower than hipBLASLt's (about 1.22 vs 1.44 PFLOP/s), which cancels the saving inside
-    the config-5 stack (150.5 vs 149.6 ms per step with and without it)."""
+    Against the norm kernel, the library's GEMM and the SwiGLU kernel, at 2048 -> 11264
+    columns: 12.4 and 29.2 us for 16 rows, 54 and 58 for 1100, 162 and 188 for 4096, 617
+    and 645 for 16384 (the GEMM core is slower than the library's, 1.2 against 1.4 PFLOP/s,
+    and the two elementwise passes make up for it)."""
     return _proj(x, w_gate_up, True, float(eps))
 
 

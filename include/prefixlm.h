@@ -388,7 +388,8 @@ int32_t prefixlm_version(void);
  * create one, pass it in the `timer` field of the args of the calls to time, read it,
  * destroy it. A timer must not be used by two threads at once. Kernel ids:
  * 0 fwd work list, 1 fwd, 2 fwd padding, 3 bwd work lists, 4 bwd pre-pass (delta),
- * 5 bwd dK/dV, 6 bwd padding, 7 bwd dQ. */
+ * 5 bwd dK/dV, 6 bwd padding, 7 bwd dQ. 2 and 6 have no launches: kernels 1 and 4 write the
+ * padding rows. 0 has none where a small forward needs no list. */
 #define PREFIXLM_NUM_KERNELS 8
 void* prefixlm_timer_create(void);          /* NULL if out of host memory */
 void prefixlm_timer_destroy(void* timer);
