@@ -30,7 +30,7 @@ constexpr int D = 128;
 constexpr int NT = 256;
 constexpr int GROUPS = NT / 16;      // keys in flight per workgroup step (x kUnroll)
 constexpr int kUnroll = 4;
-constexpr int kStep = GROUPS * kUnroll;   // keys per workgroup step
+constexpr int kStep = GROUPS * kUnroll;   // keys per step of a workgroup of NT threads
 constexpr int kPart = D + 4;         // floats per partial: max (log2 units), sum, 2 unused, o[D]
 static_assert(kPart % 4 == 0, "partials keep o 16-byte aligned");
 
@@ -86,9 +86,14 @@ __device__ __forceinline__ u32x4 load_once(const bf16* p) {
 // against 285 with plain loads and 322 for fixed 512-key splits, plain loads and an append
 // launch. Loading the next 64 keys at the end of a step instead of at its start is worth 2%;
 // doing it before the step's P V, or the heads as the fastest grid index, changes nothing.
-__global__ __launch_bounds__(NT) void decode_kernel(Params P) {
-  __shared__ float s_m[NT / 64], s_l[NT / 64];
-  __shared__ f32x4 s_o[NT / 64][D / 4];
+// NTH = 512 for calls of one split and few workgroups, where a CU would hold four waves only and
+// the walk is a chain of memory round trips: twice the keys per step (16 pairs x 256 keys 5.5 ->
+// 4.9 us, 256 pairs x 512 13.6 -> 10.9).
+template <int NTH>
+__global__ __launch_bounds__(NTH) void decode_kernel(Params P) {
+  constexpr int NWAVE = NTH / 64, GROUPS = NTH / 16, kStep = GROUPS * kUnroll;   // keys per workgroup step
+  __shared__ float s_m[NWAVE], s_l[NWAVE];
+  __shared__ f32x4 s_o[NWAVE][D / 4];
   const int split = blockIdx.x % P.nsplit;
   const int bh = blockIdx.x / P.nsplit;
   const int h = bh % P.H, b = bh / P.H;
@@ -190,11 +195,13 @@ __global__ __launch_bounds__(NT) void decode_kernel(Params P) {
   }
   __syncthreads();
   if (tid < D / 4) {
-    M = fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]));
+    M = s_m[0];
+#pragma unroll
+    for (int g = 1; g < NWAVE; ++g) M = fmaxf(M, s_m[g]);
     float L = 0.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int g = 0; g < NT / 64; ++g) {
+    for (int g = 0; g < NWAVE; ++g) {
       const float wgt = s_m[g] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[g] - M);
       L += wgt * s_l[g];
       acc += wgt * s_o[g][tid];

@@ -1084,11 +1084,11 @@ static int64_t kv_nsplit(int64_t B, int S, int64_t H, int64_t Smax) {
     // and two splits each of 512 keys or more, which even out ragged lengths (1024 pairs x
     // 4096: 272 us at one split, 263 at two, 266 at four; 2048 pairs x 256: 41 at one, 46 at
     // two).
-    // Caches of up to 256 rows: one split, whose keys take less time than the combine's launch
-    // (16 pairs x 128 keys 4.3 us, 6.9 with two splits; x 256 6.9 and 7.1 with four; x 384 9.3
-    // and 7.2).
+    // Caches of up to 384 rows: one split, whose keys take less time than the combine's launch
+    // (16 pairs x 128 keys 4.2 us, 6.9 with two splits; x 384 5.8 and 7.2; 128 pairs x 384 8.4
+    // and 10.1; 32 pairs x 512 8.6 and 7.4).
     const int64_t units = B * H;
-    if (units <= 128 && Smax <= 256) return 1;
+    if (units <= 128 && Smax <= 384) return 1;
     if (units <= 128)
       return std::max<int64_t>(1, std::min({(512 + units - 1) / units, (Smax + kvc::kStep - 1) / kvc::kStep,
                                             (int64_t)kvc::kMaxSplits}));
@@ -1248,8 +1248,13 @@ int prefixlm_kvcache_fwd(const prefixlm_kvcache_args* a, void* stream_) {
   {
     const int64_t units = (int64_t)B * H * P.nsplit, nblk = S == 1 ? units : (units + 7) / 8 * 8 * P.nqb;
     if (nblk > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "grid too large");
-    if (S == 1)
-      hipLaunchKernelGGL(kvc::decode_kernel, dim3((unsigned)nblk), dim3(kvc::NT), 0, stream, P);
+    if (S == 1 && P.nsplit == 1 && (int64_t)B * H <= 256 && Smax > kvc::kStep)
+      // one workgroup per CU at most: eight waves each (256 pairs x 256 keys 7.5 -> 6.4 us, x 768
+      // 18.5 -> 15.8; 512 pairs x 192 8.7 and 9.1; x 64 keys, one step of four waves, 4.0 and 4.4;
+      // sixteen waves are slower than eight everywhere below 512 keys)
+      hipLaunchKernelGGL(kvc::decode_kernel<512>, dim3((unsigned)nblk), dim3(512), 0, stream, P);
+    else if (S == 1)
+      hipLaunchKernelGGL(kvc::decode_kernel<kvc::NT>, dim3((unsigned)nblk), dim3(kvc::NT), 0, stream, P);
     else if (ext_qw(S) == 1)
       hipLaunchKernelGGL(kvc::extend_kernel<1>, dim3((unsigned)nblk), dim3(kvc::NT), kvc::ExtGeo<1>::LDS_BYTES, stream, P);
     else if (ext_qw(S) == 2)
