@@ -217,6 +217,11 @@ __global__ __launch_bounds__(NTH, 1) void proj_gemm_kernel(Params P) {
         if (ks + 1 < KS) {
           rd(buf, ks + 1, set ^ 1);
         } else {
+          // this step's operands are in registers before the barrier after which other waves load
+          // into this buffer: the branches of advance() end the block here, and the compiler would
+          // otherwise move reads used only after them past the barrier
+#pragma unroll
+          for (int m = 1; m < MI; ++m) settle(__builtin_bit_cast(u32x4, bfr[set][m]));
           stage_barrier();
           advance();
           rd(buf ^ 1, 0, set ^ 1);

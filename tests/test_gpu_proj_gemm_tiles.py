@@ -36,3 +36,13 @@ def test_proj_gemm_tiles(M, K, N, swiglu):
         bound = 1.02 * 2.0 ** -8 * ref.abs() + 2.0 ** -18 * size + 1e-12
         worst = ((y - ref).abs() / bound).max().item()
         assert worst <= 1.0, (norm, worst)
+
+
+@pytest.mark.parametrize("M,K,N", [(3778, 2048, 11264), (1537, 128, 8192), (1150, 2048, 16384)])
+def test_repeats_over_several_tiles_per_workgroup(M, K, N):
+    """A workgroup's stages of successive tiles share two buffers: every pass gives the same bits."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).to(DEV)
+    first = proj_gemm(x, w, True, True, EPS)
+    assert all(torch.equal(proj_gemm(x, w, True, True, EPS), first) for _ in range(40))
