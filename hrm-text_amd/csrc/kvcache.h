@@ -56,6 +56,18 @@ __device__ __forceinline__ int cache_len(const Params& P, int b) {
   return P.seqlens ? P.seqlens[b] : P.seqlen_const;
 }
 
+// The keys that query i sees of a cache row of length len: [0, n)
+__device__ __forceinline__ int keys_seen(const Params& P, int len, int i) {
+  const int lk = min(P.Smax, len + P.s_new);
+  return P.causal ? min(lk, len + P.s_new - P.S + i + 1) : lk;
+}
+// 1 / (sum of the weights) of a query that sees n keys. Without keys its row is 0; with keys whose
+// scores are all -inf the sum is 0 and the row NaN, as softmax gives it.
+__device__ __forceinline__ float row_inv(int n, float sum) { return n > 0 ? 1.f / sum : 0.f; }
+// What exponents are taken against: a running max of -inf (no key yet, or only keys whose score is
+// -inf) would turn exp2(-inf - max) into NaN where the weight is 0.
+__device__ __forceinline__ float max_ref(float m) { return m == -INFINITY ? 0.f : m; }
+
 // thread = 16-byte chunk of one (b, i, h) row of k and of v
 __global__ __launch_bounds__(256) void append_kernel(Params P) {
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -140,7 +152,7 @@ __global__ __launch_bounds__(NTH) void decode_kernel(Params P) {
     *reinterpret_cast<u32x4*>(P.kc + b * P.kc_sb + h * P.kc_sh + len * P.kc_ss + 8 * g16) = kn;
     *reinterpret_cast<u32x4*>(P.vc + b * P.vc_sb + h * P.vc_sh + len * P.vc_ss + 8 * g16) = vn;
     m = dot(kn);
-    l = __builtin_amdgcn_exp2f(m - m);
+    l = __builtin_amdgcn_exp2f(m - max_ref(m));   // 1, or 0 for a score of -inf
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       o[2 * e] = l * bf16lo(vn[e]);
@@ -154,13 +166,13 @@ __global__ __launch_bounds__(NTH) void decode_kernel(Params P) {
       s[u] = (j0 + u * GROUPS < k1) ? dot(kw[u]) : -INFINITY;
       mx = fmaxf(mx, s[u]);
     }
-    const float alpha = __builtin_amdgcn_exp2f(m - mx);   // m = -inf at first: 0
+    const float ref = max_ref(mx), alpha = __builtin_amdgcn_exp2f(m - ref);   // m = -inf at first: 0
     l *= alpha;
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] *= alpha;
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-      const float p = __builtin_amdgcn_exp2f(s[u] - mx);
+      const float p = __builtin_amdgcn_exp2f(s[u] - ref);
       l += p;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -207,7 +219,7 @@ __global__ __launch_bounds__(NTH) void decode_kernel(Params P) {
       acc += wgt * s_o[g][tid];
     }
     if (P.nsplit == 1) {
-      const float inv = L > 0.f ? 1.f / L : 0.f;
+      const float inv = row_inv(keys_seen(P, len, 0), L);
       *reinterpret_cast<bf16x4*>(P.out + b * P.o_sb + h * P.o_sh + 4 * tid) =
           cvt4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
       return;
@@ -639,7 +651,7 @@ __global__ __launch_bounds__(256) void combine_kernel(Params P) {
   for (int m = 1; m < 64; m <<= 1) L += __shfl_xor(L, m);
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc[e] += wave_xor32(acc[e]);
-  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const float inv = row_inv(keys_seen(P, cache_len(P, b), i), L);
   if (lane < 32)
     *reinterpret_cast<bf16x4*>(P.out + b * P.o_sb + i * P.o_ss + h * P.o_sh + 4 * lane) =
         cvt4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);

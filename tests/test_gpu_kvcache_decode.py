@@ -41,3 +41,31 @@ def test_decode_lengths(B, H, Smax):
 
 def test_decode_shared_cache_row():
     _run(3, 4, 300, [200, 200, 200], shared=True)
+
+
+@pytest.mark.parametrize("value", [float("-inf"), -3.3e38])
+@pytest.mark.parametrize("where", ["new", "cached", "all"])
+@pytest.mark.parametrize("B,H,Smax", [(10, 4, 700), (130, 2, 129), (2, 2, 300)])
+def test_decode_keys_of_score_minus_infinity(B, H, Smax, where, value):
+    """Keys whose score is -inf weigh nothing: the new one, every cached one of the first two key
+    steps, or all of a row's, which alone makes its output NaN. A row without keys is 0."""
+    print(f"[case] decode -inf B={B} Smax={Smax} {where} {value}", flush=True)
+    g = torch.Generator().manual_seed(B + Smax)
+    mk = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)  # noqa: E731
+    q, k, v, kc, vc = mk(B, 1, H, 128), mk(B, 1, H, 128), mk(B, 1, H, 128), mk(B, Smax, H, 128), mk(B, Smax, H, 128)
+    q[..., 7] = 16.0                              # 16 * -3.3e38 is past the range of fp32, scaled or not
+    if where != "cached":
+        k[..., 7] = value
+    if where != "new":
+        kc[:, :128 if where == "cached" else Smax, :, 7] = value
+    edges = [1, 16, 17, 63, 64, 65, 128, Smax // 2, Smax - 2, 0]
+    lens = torch.tensor([min(edges[(i + (where == "cached")) % 10], Smax - 1) for i in range(B)], dtype=torch.int32)
+    ref, _, _ = kvcache_attention(q, kc, vc, k, v, lens)
+    assert torch.isnan(ref).any() == (where == "all" or (where == "new" and 0 in lens.tolist()))
+    d = [t.to(DEV) for t in (q, k, v, kc, vc)]
+    out = flash_attn_with_kvcache(d[0], d[3], d[4], k=d[1], v=d[2], cache_seqlens=lens.to(DEV)).float().cpu()
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    err, tol = (out - ref).abs(), ref.abs() * 2.0 ** -8 + 5.0 * 2.0 ** -14
+    assert (torch.isnan(ref) | (err <= tol)).all()
+    none = flash_attn_with_kvcache(d[0], d[3], d[4], cache_seqlens=torch.zeros_like(lens).to(DEV))
+    assert (none == 0).all()
