@@ -304,8 +304,8 @@ __device__ __forceinline__ void extend_block_valu(const Params& P, int b, int h,
 #pragma unroll
       for (int e = 0; e < 4; ++e) s += q[2 * e] * bf16lo(kv[e]) + q[2 * e + 1] * bf16hi(kv[e]);
       s = row16_sum(s);
-      const float mx = fmaxf(m, s);
-      const float alpha = __builtin_amdgcn_exp2f(m - mx), p = __builtin_amdgcn_exp2f(s - mx);
+      const float mx = fmaxf(m, s), ref = max_ref(mx);
+      const float alpha = __builtin_amdgcn_exp2f(m - ref), p = __builtin_amdgcn_exp2f(s - ref);
       m = mx;
       l = l * alpha + p;
 #pragma unroll
@@ -315,7 +315,7 @@ __device__ __forceinline__ void extend_block_valu(const Params& P, int b, int h,
       }
     }
     if (P.nsplit == 1) {
-      const float inv = l > 0.f ? 1.f / l : 0.f;
+      const float inv = row_inv(kmax(i), l);
       *reinterpret_cast<bf16x8*>(P.out + b * P.o_sb + i * P.o_ss + h * P.o_sh + 8 * g16) =
           cvt8(o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv, o[4] * inv, o[5] * inv, o[6] * inv, o[7] * inv);
     } else {
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(NT, 2) void extend_kernel(Params P) {
   const int lk = min(P.Smax, len + P.s_new);      // keys in the cache after the append
   const int q0 = qb * 32 * QW;
   // query i sees keys [0, kmax(i))
-  auto kmax = [&](int i) { return P.causal ? min(lk, len + P.s_new - P.S + i + 1) : lk; };
+  auto kmax = [&](int i) { return keys_seen(P, len, i); };
   const int per = ((lk + P.nsplit - 1) / P.nsplit + TK - 1) / TK * TK;   // keys per split, whole tiles
   const int k0 = split * per;
   const int k1 = min(kmax(min(P.S, q0 + 32 * QW) - 1), k0 + per);
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(NT, 2) void extend_kernel(Params P) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
         }
-        const float m_use = m_run == -INFINITY ? 0.f : m_run;
+        const float m_use = max_ref(m_run);
         bf16x8 ph[2], pl[2];
         float ps = 0.f;
 #pragma unroll
@@ -579,7 +579,7 @@ __global__ __launch_bounds__(NT, 2) void extend_kernel(Params P) {
   if (kw == 0 && active) {
     if (P.nsplit == 1) {
       // whole rows through LDS
-      const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+      const float inv = row_inv(kmax(min(qrow, P.S - 1)), l_run);
       char* wl = smem + qw * OUT_WAVE_BYTES;
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)

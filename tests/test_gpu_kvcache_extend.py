@@ -107,3 +107,32 @@ def test_extend_non_finite_values(S):
     want = torch.full_like(out[:, bad:], float("inf"))
     want[..., 5] = float("-inf")
     assert torch.equal(out[:, bad:], want)
+
+
+@pytest.mark.parametrize("value_inf", [False, True])
+@pytest.mark.parametrize("where", ["first", "all"])
+@pytest.mark.parametrize("B,S,Smax", [(2, 6, 400), (2, 50, 400), (2, 100, 400), (70, 6, 60)])
+def test_extend_keys_of_score_minus_infinity(B, S, Smax, where, value_inf):
+    """Cached keys whose score is -inf weigh nothing, with and without a value row that is infinite
+    (seen by the last three queries only); a query whose keys are all such is NaN."""
+    print(f"[case] extend -inf B={B} S={S} {where} {value_inf}", flush=True)
+    H = 2
+    q, k, v, kc, vc = _inputs(B, S, H, Smax, 23)
+    lens = torch.full((B,), min(150, Smax - S), dtype=torch.int32)
+    lens[1] = Smax - S
+    q[..., 3] = 2.0
+    kc[:, :40, :, 3] = float("-inf")
+    if where == "all":
+        kc[1, ..., 3] = k[1, :S // 2, :, 3] = float("-inf")
+    last = S - 3
+    if value_inf:
+        v[:, last] = float("inf")
+    ref, _, _ = kvcache_attention(q, kc, vc, k, v.nan_to_num(posinf=0.0), lens, True)
+    d = [t.to(DEV) for t in (q, k, v, kc, vc)]
+    out = flash_attn_with_kvcache(d[0], d[3], d[4], k=d[1], v=d[2], cache_seqlens=lens.to(DEV), causal=True).float().cpu()
+    rows = slice(0, last) if value_inf else slice(0, S)
+    got, ref = out[:, rows], ref[:, rows]
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.isnan(ref).any() == (where == "all")
+    _check(got.nan_to_num(), ref.nan_to_num(), 5.0)
+    if value_inf:
+        assert (out[:, last:] == float("inf")).all()
