@@ -4,8 +4,8 @@ and key splits, with rows that fall past the cache, cached-only calls, strided a
 caches, and non-finite values.
 
 Tolerance per element: half a bf16 ulp of the reference (2^-8 |ref|, the output's own
-rounding) plus 2^-14 max|V|: P enters P V as two bf16 terms, which leaves at most 2^-17 of
-each probability, and fp32 sums of up to 1500 terms in another order stay below 2^-15."""
+rounding) plus 2^-14 max|V|: P enters P V with its fp32 bits, and fp32 sums of up to 1500 terms in
+another order stay below 2^-15."""
 import pytest
 import torch
 
@@ -136,3 +136,28 @@ def test_extend_keys_of_score_minus_infinity(B, S, Smax, where, value_inf):
     _check(got.nan_to_num(), ref.nan_to_num(), 5.0)
     if value_inf:
         assert (out[:, last:] == float("inf")).all()
+
+
+@pytest.mark.parametrize("S", [2, 40, 100])
+@pytest.mark.parametrize("Smax,at", [(128, (0, 1, 2)), (1000, (700, 5, 6)), (1000, (0, 5, 800))])
+def test_extend_keeps_the_bits_of_the_probabilities(S, Smax, at):
+    """Three keys count: one of weight 1 and value 0, and two of nearly the same weight, 0.4 to 0.9,
+    with values +1 and -1, whose difference of about 1e-4 is the output.
+
+    Bound: half a bf16 ulp of the result plus 2^-21, four times what fp32 weights leave (an exponent
+    below 2 in magnitude, rounded twice, and exp2 to 1 ulp, each weight less than 0.4 of the sum:
+    2 * 0.4 * 2^-22.5). Weights of 16 bits are off by up to 2^-18 each."""
+    B, H = 2, 5
+    q, k, v, kc, vc = (torch.zeros(B, n, H, 128, dtype=torch.bfloat16) for n in (S, S, S, Smax, Smax))
+    g = torch.Generator().manual_seed(S + Smax)
+    q[..., 0] = (0.08 + 0.6 * torch.rand(B, S, H, generator=g)).to(torch.bfloat16)
+    kc[..., 0], k[..., 0] = -3e4, -3e4
+    for j, a, x in zip(at, (16.0, 1.0, 1.0078125), (0.0, 1.0, -1.0)):
+        kc[:, j, :, 0], vc[:, j] = a, x
+    lens = torch.full((B,), Smax - S, dtype=torch.int32)
+    d = [t.to(DEV) for t in (q, k, v, kc, vc)]
+    out = flash_attn_with_kvcache(d[0], d[3], d[4], k=d[1], v=d[2], cache_seqlens=lens.to(DEV), causal=True).double().cpu()
+    w = torch.softmax(q[..., :1].double() * torch.tensor([16.0, 1.0, 1.0078125], dtype=torch.float64) / 128 ** 0.5, -1)
+    ref = (w[..., 1] - w[..., 2]).unsqueeze(-1)
+    worst = ((out - ref).abs() - ref.abs() * 2.0 ** -8).max().item()
+    assert worst <= 2.0 ** -21, f"{worst:.3e}"
