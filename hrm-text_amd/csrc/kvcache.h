@@ -280,8 +280,10 @@ __device__ __forceinline__ u16x2 max_mag(u16x2 m, const u32x4& w) {
 
 // Queries [q0, q1) over keys [k0, k1) without the matrix cores: a 16-lane group per query,
 // key by key. For blocks whose values hold an infinity or NaN: in P V on the matrix cores
-// hi * inf + lo * inf is NaN where the signs differ, and 0 * inf would reach queries that
-// must not see the key; here a query touches only the keys it sees.
+// 0 * inf would reach queries that must not see the key; here a query touches only the keys it
+// sees. And for blocks with such a score: the matrix cores sum q k before the softmax scale, and
+// that sum can pass fp32's range (keys of the type's lowest value) where the scaled one here does
+// not.
 template <class KMax, class KRow, class VRow>
 __device__ __forceinline__ void extend_block_valu(const Params& P, int b, int h, int split, int q0, int q1, int k0,
                                                   int k1, KMax kmax, KRow k_row, VRow v_row) {
@@ -333,7 +335,7 @@ __global__ __launch_bounds__(NT, 2) void extend_kernel(Params P) {
   using G = ExtGeo<QW>;
   constexpr int KW = G::KW, TK = G::TK, TILE = G::TILE, NS = D / 16, NP = TK / 16;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  __shared__ int bad;   // some value row holds an infinity or NaN
+  __shared__ int bad;   // some value row holds an infinity or NaN, or some score is one
 
   // unit u = (b, h, split); its query blocks sit 8 grid indices apart, on one XCD
   const int qb = (blockIdx.x >> 3) % P.nqb;
@@ -530,11 +532,6 @@ __global__ __launch_bounds__(NT, 2) void extend_kernel(Params P) {
       if (t + 1 < nt) store_kv(G::NBUF == 2 ? buf ^ 1 : 0);
       __syncthreads();
     }
-    if (bad) {
-      extend_block_valu(P, b, h, split, q0, min(P.S, q0 + 32 * QW), k0, k1, kmax, k_row, v_row);
-      append_share();
-      return;
-    }
     l_run = halves_sum(l_run);
     // the KW waves of one query block: waves kw > 0 hand theirs to wave kw = 0
     if (KW > 1) {
@@ -581,7 +578,17 @@ __global__ __launch_bounds__(NT, 2) void extend_kernel(Params P) {
         }
         l_run = L;
       }
-      __syncthreads();
+    }
+    // a score past the range upwards leaves NaN; one past it downwards (raw below -3.4e38) only
+    // counts where every key that the query sees here scores about as low
+    if (kw == 0 && active && min(k1, kmax(min(qrow, P.S - 1))) > k0 &&
+        (l_run != l_run || m_run < 200.f - 3e38f * fabsf(P.scale_log2)))
+      bad = 1;
+    __syncthreads();
+    if (bad) {
+      extend_block_valu(P, b, h, split, q0, min(P.S, q0 + 32 * QW), k0, k1, kmax, k_row, v_row);
+      append_share();
+      return;
     }
   }
   if (kw == 0 && active) {

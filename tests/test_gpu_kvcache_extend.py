@@ -161,3 +161,25 @@ def test_extend_keeps_the_bits_of_the_probabilities(S, Smax, at):
     ref = (w[..., 1] - w[..., 2]).unsqueeze(-1)
     worst = ((out - ref).abs() - ref.abs() * 2.0 ** -8).max().item()
     assert worst <= 2.0 ** -21, f"{worst:.3e}"
+
+
+@pytest.mark.parametrize("scale", [None, -0.05])
+@pytest.mark.parametrize("S", [1, 2, 40, 100])
+def test_extend_scores_past_the_range_before_the_scale(S, scale):
+    """Keys of about the type's lowest value: q k is -6e38, infinite in fp32, and -5e37 with the
+    softmax scale. Every key of the first sequence scores the same, so its output is the mean of
+    the values that a query sees; the second sequence sees one other key, which takes it all."""
+    B, H, Smax = 2, 3, 300
+    q, k, v, kc, vc = _inputs(B, S, H, Smax, 31)
+    q.zero_(), k.zero_(), kc.zero_()
+    q[..., 0] = 2.0 if scale is None else -2.0
+    kc[..., 0] = k[..., 0] = -3e38
+    kc[1, 7, :, 0] = 0.0
+    lens = torch.tensor([130, 200], dtype=torch.int32)
+    d = [t.to(DEV) for t in (q, k, v, kc, vc)]
+    out = flash_attn_with_kvcache(d[0], d[3], d[4], k=d[1], v=d[2], cache_seqlens=lens.to(DEV), causal=True,
+                                  softmax_scale=scale).float().cpu()
+    rows = torch.cat((vc[0, :130], v[0])).double()
+    mean = torch.stack([rows[:130 + i + 1].mean(0) for i in range(S)])
+    _check(out[0], mean.float(), 5.0)
+    assert torch.equal(out[1], vc[1, 7].float().expand(S, H, 128))
