@@ -201,6 +201,21 @@ struct Batch {
     }
     a.timer = g_timer.load();
   }
+  // whether the metadata that a backward got back is what parse accepted
+  bool restored(const Tensor& like) const {
+    if (!meta(pre, like) || !meta(cau, like) || !meta(cu, like)) return false;
+    if (plan.defined() && (!meta(plan, like) || plan.dim() != 1 || !aligned(plan, 256))) return false;
+    for (const Scalar* s : {&total, &nseq, &mp, &mc, &ma, &dsb}) {
+      if (s == &dsb && !has_dsb) continue;
+      const Tensor& t = s->t;
+      if (!t.defined() || !t.device().is_cpu() || t.numel() != 1) return false;
+      const bool same = t.scalar_type() == at::kLong  ? *t.const_data_ptr<int64_t>() == s->v
+                        : t.scalar_type() == at::kInt ? *t.const_data_ptr<int32_t>() == s->v
+                                                      : false;
+      if (!same) return false;
+    }
+    return true;
+  }
   static Tensor scalar(const Scalar& s) { return s.t.defined() ? s.t : at::scalar_tensor(s.v, at::kLong); }
   // saved with the call: the tensors that the Python function saves, in its order (an in-place
   // change is noticed, and a recomputation may take either path), and the values
@@ -368,12 +383,35 @@ void attn_backward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
 }
 
 // A backward runs the kernels directly on plain tensors; one that is recorded itself, or
-// under a mode or a batched gradient, is the custom op's.
+// under a mode or a batched gradient, is the custom op's. So is one whose saved tensors are not
+// those the forward saved: a saved-tensors hook may give back another dtype, shape, layout or
+// device, and the kernels get raw pointers. The custom op copies or refuses such operands.
 bool direct_backward(const variable_list& saved, const Tensor& grad, const Tensor& like, int64_t* cap) {
   if (at::GradMode::is_enabled() || !plain_state() || !ds_cap(like, cap)) return false;
   for (const Tensor& t : saved)
     if (t.defined() && !plain_tensor(t, !t.device().is_cpu())) return false;
-  return plain_tensor(grad) && grad.scalar_type() == at::kBFloat16 && grad.device() == like.device();
+  return plain_tensor(grad) && grad.scalar_type() == at::kBFloat16 && plain_tensor(like) &&
+         grad.device() == like.device();
+}
+bool is_array(const Tensor& x, at::ScalarType dt, at::IntArrayRef sizes, const Tensor& like) {
+  return x.defined() && x.scalar_type() == dt && x.sizes() == sizes && x.device() == like.device();
+}
+// out, lse, out_lo and q_amax as attn_forward makes them for the [T, H, D] of `sizes`
+bool attn_saved(const Tensor& out, const Tensor& lse, const Tensor& out_lo, const Tensor& q_amax, at::IntArrayRef sizes,
+                const Tensor& like) {
+  return is_array(out, at::kBFloat16, sizes, like) && operand_layout(out) &&
+         is_array(lse, at::kFloat, {sizes[1], sizes[0]}, like) && lse.is_contiguous() &&
+         is_array(out_lo, at::kChar, sizes, like) && out_lo.stride(2) == 1 && out_lo.stride(0) % 16 == 0 &&
+         out_lo.stride(1) % 16 == 0 && aligned(out_lo, 16) &&
+         is_array(q_amax, at::kFloat, {(int64_t)lib.q_amax_count(sizes[0], sizes[1])}, like) && q_amax.is_contiguous();
+}
+// what the fused layer reads of cos and sin [T, 128]
+bool rope_tables(const Tensor& cos, const Tensor& sin, int64_t T, const Tensor& like) {
+  for (const Tensor& c : {cos, sin})
+    if (!is_array(c, at::kFloat, {T, 128}, like) || c.stride(1) != 1 || c.stride(0) % 4 ||
+        c.stride(0) != cos.stride(0) || !aligned(c, 16))
+      return false;
+  return true;
 }
 
 struct Varlen : torch::autograd::Function<Varlen> {
@@ -389,7 +427,11 @@ struct Varlen : torch::autograd::Function<Varlen> {
     const Batch b = Batch::restore(s, 7, ctx);
     int64_t cap = 0;
     variable_list g;
-    if (direct_backward(s, grads[0], s[0], &cap)) {
+    bool direct = direct_backward(s, grads[0], s[0], &cap) &&
+                  attn_saved(s[3], s[4], s[5], s[6], grads[0].sizes(), s[0]) && b.restored(s[0]);
+    for (int i = 0; i < 3 && direct; ++i)
+      direct = is_array(s[i], at::kBFloat16, grads[0].sizes(), s[0]) && operand_layout(s[i]);
+    if (direct) {
       const c10::DeviceGuard guard(s[0].device());
       const Tensor dout = as_operand(grads[0]);
       for (int i = 0; i < 3; ++i) g.push_back(empty_like_on(s[0], s[0].sizes(), at::kBFloat16));
@@ -446,10 +488,17 @@ struct Layer : torch::autograd::Function<Layer> {
     const Batch b = Batch::restore(s, 8, ctx);
     int64_t cap = 0;
     Tensor dg;
-    if (direct_backward(s, grads[0], s[0], &cap)) {
-      const c10::DeviceGuard guard(s[0].device());
-      const Tensor &gqkv = s[0], &qk = s[1];
-      const int64_t H = gqkv.size(1) / 4;
+    const Tensor &gqkv = s[0], &qk = s[1];
+    bool direct = direct_backward(s, grads[0], gqkv, &cap) && b.restored(gqkv);
+    if (direct) {
+      const int64_t T = grads[0].size(0), H = grads[0].size(1);
+      direct = is_array(gqkv, at::kBFloat16, {T, 4 * H, 128}, gqkv) && gqkv.is_contiguous() && aligned(gqkv, 16) &&
+               is_array(qk, at::kBFloat16, {T, 2 * H, 128}, gqkv) && qk.is_contiguous() && aligned(qk, 16) &&
+               attn_saved(s[2], s[3], s[4], s[5], grads[0].sizes(), gqkv) && rope_tables(s[6], s[7], T, gqkv);
+    }
+    if (direct) {
+      const int64_t H = grads[0].size(1);
+      const c10::DeviceGuard guard(gqkv.device());
       const Tensor dy = grads[0].contiguous();
       dg = empty_like_on(gqkv, gqkv.sizes(), at::kBFloat16);
       attn_backward(qk.narrow(1, 0, H), qk.narrow(1, H, H), gqkv.narrow(1, 3 * H, H), s[2], s[3], s[4], s[5], dy,
@@ -512,7 +561,8 @@ struct Swiglu : torch::autograd::Function<Swiglu> {
     const Tensor& gu = s[0];
     int64_t cap = 0;
     Tensor g2;
-    if (direct_backward(s, grads[0], gu, &cap) && (g2 = rows_view(gu)).defined()) {
+    if (direct_backward(s, grads[0], gu, &cap) && (g2 = rows_view(gu)).defined() &&
+        g2.size(1) == 2 * grads[0].size(-1) && gu.numel() == 2 * grads[0].numel()) {
       const c10::DeviceGuard guard(gu.device());
       const Tensor d2 = rows_of(grads[0]);
       const Tensor dgu = empty_like_on(gu, gu.sizes(), at::kBFloat16);
@@ -559,7 +609,8 @@ struct RmsNorm : torch::autograd::Function<RmsNorm> {
     const Tensor& x = s[0];
     int64_t cap = 0;
     Tensor x2;
-    if (direct_backward(s, grads[0], x, &cap) && (x2 = rows_view(x)).defined()) {
+    if (direct_backward(s, grads[0], x, &cap) && (x2 = rows_view(x)).defined() && x.sizes() == grads[0].sizes() &&
+        is_array(s[1], at::kFloat, {x2.size(0)}, x) && s[1].is_contiguous()) {
       const c10::DeviceGuard guard(x.device());
       const Tensor d2 = rows_of(grads[0]);
       const Tensor dx = empty_like_on(x, x.sizes(), at::kBFloat16);
@@ -616,11 +667,7 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (g.scalar_type() != at::kBFloat16 || g.dim() != 3 || g.size(1) % 4 || g.size(2) != 128 || g.numel() == 0 ||
       !g.is_contiguous() || !aligned(g, 16))
     return none();
-  for (const Tensor& c : {cos, sin})
-    if (c.scalar_type() != at::kFloat || c.dim() != 2 || c.size(0) != g.size(0) || c.size(1) != 128 ||
-        c.stride(1) != 1 || c.stride(0) % 4 || c.stride(0) != cos.stride(0) || !aligned(c, 16) ||
-        c.device() != g.device() || wants_grad(c))
-      return none();
+  if (!rope_tables(cos, sin, g.size(0), g) || wants_grad(cos) || wants_grad(sin)) return none();
   if (!b.parse(a + 3, g, g.size(2))) return none();
   Tensor y;
   {

@@ -150,3 +150,79 @@ def test_hooks_checkpoint_and_other_streams(path):
     assert torch.equal(got, want)
     with torch.inference_mode():
         assert torch.equal(f(q.detach()), out.detach())
+
+
+def _wide(t):
+    """t's values in rows of twice the length."""
+    return torch.cat((t, t), -1)[..., :t.shape[-1]]
+
+
+def _shifted(t):
+    """t's values one element off its alignment."""
+    return torch.cat((t.flatten()[:1], t.flatten()))[1:].view(t.shape)
+
+
+# which saved tensor (by dtype and number of dimensions, the n-th such), what a hook gives back for
+# it, and what the backward then does: the same gradients, or this error
+HOOKS = {
+    "q_fp32": ("varlen", (torch.bfloat16, 3, 0), lambda t: t.float(), TypeError),
+    "k_cpu": ("varlen", (torch.bfloat16, 3, 1), lambda t: t.cpu(), ValueError),
+    "v_off_alignment": ("varlen", (torch.bfloat16, 3, 2), _shifted, RuntimeError),
+    "out_wide": ("varlen", (torch.bfloat16, 3, 3), _wide, None),
+    "lse_transposed": ("varlen", (torch.float32, 2, 0), lambda t: t.t().contiguous().t(), None),
+    "lse_double": ("varlen", (torch.float32, 2, 0), lambda t: t.double(), ValueError),
+    "residual_strided": ("varlen", (torch.int8, 3, 0), lambda t: torch.stack((t, t), -1)[..., 0], None),
+    "residual_short": ("varlen", (torch.int8, 3, 0), lambda t: t[:-1], ValueError),
+    "q_amax_short": ("varlen", (torch.float32, 1, 0), lambda t: t[:-1], ValueError),
+    "q_amax_strided": ("varlen", (torch.float32, 1, 0), lambda t: torch.stack((t, t), -1)[:, 0], None),
+    "lens_long": ("varlen", (torch.int32, 1, 0), lambda t: t.long(), None),
+    "plan_off_alignment": ("varlen", (torch.int32, 1, 3), _shifted, None),
+    "scalar_gpu": ("varlen", (torch.int64, 0, 0), lambda t: t.to(DEV), AssertionError),
+    "gqkv_wide": ("layer", (torch.bfloat16, 3, 0), _wide, None),
+    "gqkv_fp32": ("layer", (torch.bfloat16, 3, 0), lambda t: t.float(), ValueError),
+    "cos_wide": ("layer", (torch.float32, 2, 1), lambda t: torch.cat((t, t), -1)[:, :128].contiguous(), None),
+    "sin_short": ("layer", (torch.float32, 2, 2), lambda t: t[:-1], ValueError),
+    "rstd_strided": ("rms_norm", (torch.float32, 1, 0), lambda t: torch.stack((t, t), -1)[:, 0], None),
+    "rstd_short": ("rms_norm", (torch.float32, 1, 0), lambda t: t[:-1], ValueError),
+    "gu_fp32": ("swiglu", (torch.bfloat16, 2, 0), lambda t: t.float(), ValueError),
+}
+
+
+@pytest.mark.parametrize("name", HOOKS)
+def test_hooks_that_give_back_other_tensors(name, path):
+    """A saved-tensors hook may change what the backward gets: the operands are checked again, and
+    copied or refused as the custom ops do."""
+    print(f"[case] hook {name} {path}", flush=True)
+    call, which, change, error = HOOKS[name]
+    T, H = 300, 2
+    b = make_batch([60, 20], [100, 70], T, H, 128, seed=6, device=DEV)
+    info = {**b.seq_info, **plan_inputs(b.seq_tensors, b.seq_scalars, DEV)}
+    cos, sin = rotary_cos_sin(torch.arange(T, device=DEV), 128, 10000.0, 1024)
+    x, f, dy = {
+        "varlen": (b.q, lambda q: flash_attn_varlen_prefixlm(q, b.k, b.v, False, **info), b.dout),
+        "layer": (_rand(T, 4 * H, 128, seed=1), lambda g: fused_attention_layer(g, cos, sin, False, **info), b.dout),
+        "rms_norm": (_rand(40, 256, seed=1), lambda x: rms_norm(x, 1e-6), _rand(40, 256, seed=2)),
+        "swiglu": (_rand(40, 512, seed=1), swiglu, _rand(40, 256, seed=2)),
+    }[call]
+    x = x.clone().requires_grad_()
+    want, = torch.autograd.grad(f(x), x, dy)
+    seen, given = {}, []
+
+    def pack(t):
+        key = (t.dtype, t.dim())
+        n = seen.get(key, 0)
+        seen[key] = n + 1
+        return t, (*key, n) == which
+
+    def unpack(p):
+        given.append(p[1])
+        return change(p[0].detach()) if p[1] else p[0]
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        y = f(x)
+    if error is None:
+        assert torch.equal(torch.autograd.grad(y, x, dy)[0], want)
+    else:
+        with pytest.raises(error):
+            torch.autograd.grad(y, x, dy)
+    assert given.count(True) == 1
