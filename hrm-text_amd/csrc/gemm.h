@@ -394,7 +394,8 @@ __global__ __launch_bounds__(64 * NWV, 1) void proj_skinny_kernel(Params P, floa
       float s = 0.f;
 #pragma unroll
       for (int v = 0; v < NWV; ++v) s += sums[(v * MB + m) * 32 + l32];
-      rs = __builtin_amdgcn_rsqf(s / (float)P.K + eps);
+      // the caller's scales (P.rstd), or the ones found here
+      rs = P.rstd != nullptr ? P.rstd[min(row, P.M - 1)] : __builtin_amdgcn_rsqf(s / (float)P.K + eps);
       if (rstd_out != nullptr && blockIdx.x == 0 && w == 0 && hh == 0 && row < P.M) rstd_out[row] = rs;
     }
     float t[NB][RW];

@@ -972,9 +972,9 @@ static int proj_skinny_launch(const mlp::Params& P, bool sw, bool norm, float* r
 }
 static int proj_skinny(const prefixlm_proj_gemm_args* a, bool given, hipStream_t stream) {
   const mlp::Params P{static_cast<const bf16*>(a->x), static_cast<const bf16*>(a->w), static_cast<bf16*>(a->y),
-                      nullptr, a->x_stride, a->w_stride, a->y_stride, a->M, a->K, a->N, 0, 0};
+                      given ? a->rstd : nullptr, a->x_stride, a->w_stride, a->y_stride, a->M, a->K, a->N, 0, 0};
   const bool sw = a->swiglu != 0, norm = a->norm != 0;
-  float* const rstd = given ? nullptr : a->rstd;   // given ones are found again from x
+  float* const rstd = given ? nullptr : a->rstd;   // where the scales found from x go
   if (a->M <= 32) return proj_skinny_launch<1, 8>(P, sw, norm, rstd, a->eps, stream);
   if (a->M <= 64) return proj_skinny_launch<2, 8>(P, sw, norm, rstd, a->eps, stream);
   return proj_skinny_launch<4, 4>(P, sw, norm, rstd, a->eps, stream);

@@ -75,6 +75,27 @@ def test_scaled_projection(path, rows):
     _same(rms_scaled_swiglu(s, w, rstd, EPS), rms_norm_swiglu(x + r, w, EPS))
 
 
+@pytest.mark.parametrize("rows", [1, 64, 100, 128, 129])
+def test_scaled_projection_takes_the_given_scales(path, rows):
+    """Scales that are not those of x are applied as given and not written, for few rows as for
+    many. Bound per element as in the projection tests: one bf16 rounding plus fp32 accumulation."""
+    x, w = _rand(rows, 256), _rand(512, 256, seed=2)
+    _, rstd = add_rms_scales(x, torch.zeros_like(x), EPS)
+    before = rstd.clone()
+    for factor in (0.125, -2.0):
+        got = rms_scaled_swiglu(x, w, factor * rstd, EPS)
+        y = (x.double() * rstd.double().unsqueeze(1) * factor) @ w.double().t()
+        gate, up = y.chunk(2, -1)
+        want = gate * torch.sigmoid(gate) * up
+        size = x.double().abs() * rstd.double().unsqueeze(1).abs() * abs(factor) @ w.double().abs().t()
+        sg, su = size.chunk(2, -1)
+        s = torch.sigmoid(gate)
+        bound = 1.02 * 2.0 ** -8 * want.abs() + 2.0 ** -18 * ((s * (1 + gate * (1 - s)) * up).abs() * sg
+                                                             + (gate * s).abs() * su) + 1e-12
+        assert ((got.double() - want).abs() <= bound).all()
+    assert torch.equal(rstd, before)
+
+
 @pytest.mark.parametrize("fused_gemm", [False, True])
 def test_stack(fused_gemm):
     cfg = HRMStackConfig(hidden_size=256, num_heads=2, layers_per_module=2, H_cycles=1, L_cycles=2, max_seq_len=256,
