@@ -412,7 +412,7 @@ static int fwd_launch(const prefixlm_fwd_args* a, void* stream_) {
     P.o_lo = static_cast<int8_t*>(a->out_lo);
     P.lse = a->lse;
     P.gate = static_cast<const bf16*>(a->gate);
-    P.y = static_cast<bf16*>(a->out_gated);
+    P.y = gated ? static_cast<bf16*>(a->out_gated) : nullptr;   // ignored without a gate
     P.q_st = a->q_stride_t; P.q_sh = a->q_stride_h;
     P.k_st = a->k_stride_t; P.k_sh = a->k_stride_h;
     P.v_st = a->v_stride_t; P.v_sh = a->v_stride_h;

@@ -143,3 +143,34 @@ def test_config5_fused_stack_within_its_own_floor():
     print(f"[parity] cfg5 bf16 stack vs fp32 stack: fused layer {e_f:.3e}, unfused {e_u:.3e}", flush=True)
     assert torch.isfinite(out_fused).all()
     assert e_f <= max(3e-2, 1.5 * e_u)
+
+
+def test_gated_output_pointer_without_a_gate_is_ignored():
+    """C ABI: out_gated left set with gate = NULL is neither checked nor written, not even on the
+    rows past total_seqlen."""
+    import ctypes
+
+    from prefixlm import _capi
+    lib = _capi.load()
+    T, H = 300, 2
+    seq, _, _, gqkv, _ = _batch([60, 20], [100, 70], T, H, 3)
+    q, k, v = (gqkv[:, i * H:(i + 1) * H].contiguous() for i in (1, 2, 3))
+    out, lse = torch.empty_like(q), torch.empty(H, T, device=DEV)
+    untouched = torch.full((T, H, 128), 7.0, dtype=torch.bfloat16, device=DEV)
+    total, n, mp, mc, ma = (int(seq[s]) for s in ("total_seqlen", "numseqs", "max_seqlen_prefix", "max_seqlen_causal",
+                                                  "max_seqlen_all"))
+    need = lib.prefixlm_fwd_workspace_size(T, H, 128, total, n)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    st, sh = H * 128, 128
+    a = _capi.FwdArgs(
+        q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), out=out.data_ptr(), lse=lse.data_ptr(), q_stride_t=st,
+        q_stride_h=sh, k_stride_t=st, k_stride_h=sh, v_stride_t=st, v_stride_h=sh, out_stride_t=st, out_stride_h=sh,
+        prefix_lens=seq["prefix_lens"].data_ptr(), causal_lens=seq["causal_lens"].data_ptr(),
+        cu_seqlens=seq["cu_seqlens"].data_ptr(), meta_len=seq["prefix_lens"].numel(), num_tokens=T, num_heads=H,
+        head_dim=128, total_seqlen=total, numseqs=n, max_seqlen_prefix=mp, max_seqlen_causal=mc, max_seqlen_all=ma,
+        softmax_scale=128 ** -0.5, workspace=ws.data_ptr(), workspace_bytes=need, out_gated=untouched.data_ptr(),
+        out_gated_stride_t=st, out_gated_stride_h=sh)
+    _capi.check(lib.prefixlm_fwd(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "prefixlm_fwd")
+    assert (out[total:] == 0).all() and (untouched == 7.0).all()
+    want = flash_attn_varlen_prefixlm(q, k, v, False, **seq)
+    assert torch.equal(out, want)
