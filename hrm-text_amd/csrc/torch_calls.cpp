@@ -23,6 +23,7 @@
 #include <c10/core/impl/PythonDispatcherTLS.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/record_function.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -32,6 +33,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
+#include <functional>
 #include <optional>
 
 #include "prefixlm.h"
@@ -77,6 +79,20 @@ Tensor empty_like_on(const Tensor& t, at::IntArrayRef sizes, at::ScalarType dt) 
   return at::empty(sizes, t.options().dtype(dt).requires_grad(false));
 }
 int i32(bool b) { return b ? 1 : 0; }
+// The calls do not pass the dispatcher, which would show them to torch.profiler: each records the
+// name of the custom op that it stands for, with its tensors, for as long as this object lives.
+struct Recorded {
+  at::RecordFunction fn{at::RecordScope::FUNCTION};
+  Recorded(const char* op, std::initializer_list<std::reference_wrapper<const Tensor>> tensors) {
+    if (!fn.isActive()) return;
+    if (fn.needsInputs()) {
+      const std::vector<c10::IValue> in(tensors.begin(), tensors.end());
+      fn.before(op, c10::ArrayRef<const c10::IValue>(in.data(), in.size()));
+    } else {
+      fn.before(op);
+    }
+  }
+};
 
 // ---- what counts as a plain call --------------------------------------------------------
 // No mode, transform or tracer that would want to see the operators.
@@ -414,9 +430,14 @@ bool rope_tables(const Tensor& cos, const Tensor& sin, int64_t T, const Tensor& 
   return true;
 }
 
+FwdOut varlen_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Batch& b) {
+  const Recorded call("prefixlm::varlen_fwd", {q, k, v});
+  return attn_forward(q, k, v, Tensor(), b);
+}
+
 struct Varlen : torch::autograd::Function<Varlen> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Batch& b) {
-    FwdOut r = attn_forward(q, k, v, Tensor(), b);
+    FwdOut r = varlen_forward(q, k, v, b);
     variable_list s{q, k, v, r.out, r.lse, r.out_lo, r.q_amax};
     b.save(s, ctx);
     ctx->save_for_backward(std::move(s));
@@ -432,6 +453,7 @@ struct Varlen : torch::autograd::Function<Varlen> {
     for (int i = 0; i < 3 && direct; ++i)
       direct = is_array(s[i], at::kBFloat16, grads[0].sizes(), s[0]) && operand_layout(s[i]);
     if (direct) {
+      const Recorded call("prefixlm::varlen_bwd", {s[0], s[1], s[2], grads[0]});
       const c10::DeviceGuard guard(s[0].device());
       const Tensor dout = as_operand(grads[0]);
       for (int i = 0; i < 3; ++i) g.push_back(empty_like_on(s[0], s[0].sizes(), at::kBFloat16));
@@ -468,6 +490,7 @@ struct LayerOut {
 };
 LayerOut layer_forward(const Tensor& gqkv, const Tensor& cos, const Tensor& sin, const Batch& b) {
   const int64_t T = gqkv.size(0), H = gqkv.size(1) / 4, D = gqkv.size(2);
+  const Recorded call("prefixlm::attn_layer_fwd", {gqkv, cos, sin});
   LayerOut r;
   r.qk = empty_like_on(gqkv, {T, 2 * H, D}, at::kBFloat16);
   rope(gqkv.narrow(1, H, 2 * H), r.qk, cos, sin, false);
@@ -497,6 +520,7 @@ struct Layer : torch::autograd::Function<Layer> {
                attn_saved(s[2], s[3], s[4], s[5], grads[0].sizes(), gqkv) && rope_tables(s[6], s[7], T, gqkv);
     }
     if (direct) {
+      const Recorded call("prefixlm::attn_layer_bwd", {grads[0], gqkv});
       const int64_t H = grads[0].size(1);
       const c10::DeviceGuard guard(gqkv.device());
       const Tensor dy = grads[0].contiguous();
@@ -537,6 +561,7 @@ Tensor rows_of(const Tensor& x) {   // a gradient: copied where its layout does 
 }
 
 Tensor swiglu_forward(const Tensor& gu, const Tensor& g2) {
+  const Recorded call("prefixlm::swiglu_fwd", {gu});
   const int64_t rows = g2.size(0), F = g2.size(1) / 2;
   auto sizes = gu.sizes().vec();
   sizes.back() = F;
@@ -563,6 +588,7 @@ struct Swiglu : torch::autograd::Function<Swiglu> {
     Tensor g2;
     if (direct_backward(s, grads[0], gu, &cap) && (g2 = rows_view(gu)).defined() &&
         g2.size(1) == 2 * grads[0].size(-1) && gu.numel() == 2 * grads[0].numel()) {
+      const Recorded call("prefixlm::swiglu_bwd", {gu, grads[0]});
       const c10::DeviceGuard guard(gu.device());
       const Tensor d2 = rows_of(grads[0]);
       const Tensor dgu = empty_like_on(gu, gu.sizes(), at::kBFloat16);
@@ -583,6 +609,7 @@ struct Swiglu : torch::autograd::Function<Swiglu> {
 };
 
 Tensor rms_forward(const Tensor& x, const Tensor& x2, double eps, Tensor* rstd) {
+  const Recorded call("prefixlm::rms_norm_fwd", {x});
   const Tensor y = empty_like_on(x, x.sizes(), at::kBFloat16);
   *rstd = empty_like_on(x, {x2.size(0)}, at::kFloat);
   prefixlm_rmsnorm_args a{};
@@ -611,6 +638,7 @@ struct RmsNorm : torch::autograd::Function<RmsNorm> {
     Tensor x2;
     if (direct_backward(s, grads[0], x, &cap) && (x2 = rows_view(x)).defined() && x.sizes() == grads[0].sizes() &&
         is_array(s[1], at::kFloat, {x2.size(0)}, x) && s[1].is_contiguous()) {
+      const Recorded call("prefixlm::rms_norm_bwd", {x, grads[0]});
       const c10::DeviceGuard guard(x.device());
       const Tensor d2 = rows_of(grads[0]);
       const Tensor dx = empty_like_on(x, x.sizes(), at::kBFloat16);
@@ -652,7 +680,7 @@ PyObject* py_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
     pybind11::gil_scoped_release no_gil;
     const c10::DeviceGuard guard(q.device());
     out = wants_grad(q) || wants_grad(k) || wants_grad(v) ? Varlen::apply(q, k, v, b)
-                                                          : attn_forward(q, k, v, Tensor(), b).out;
+                                                          : varlen_forward(q, k, v, b).out;
   }
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
@@ -714,6 +742,7 @@ PyObject* py_kvcache(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;
+    const Recorded call("prefixlm::kvcache_attn", {q, kc, vc});
     const c10::DeviceGuard guard(q.device());
     out = empty_like_on(q, {B, S, H, D}, at::kBFloat16);
     prefixlm_kvcache_args p{};
@@ -812,6 +841,7 @@ PyObject* py_add_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::NoGradGuard no_grad;
     const Tensor x2 = rows_view(x, true), r2 = rows_view(r, true);
     if (x2.defined() && r2.defined() && x2.size(1) <= INT32_MAX) {
+      const Recorded call("prefixlm::add_rmsnorm", {x, r});
       const c10::DeviceGuard guard(x.device());
       s = empty_like_on(x, x.sizes(), at::kBFloat16);
       if (with_y) y = empty_like_on(x, x.sizes(), at::kBFloat16);
@@ -871,10 +901,13 @@ Tensor projection(const Tensor& x, const Tensor& w, const Tensor& scales, bool s
   p.swiglu = i32(sw);
   p.norm = i32(norm);
   p.eps = (float)eps;
-  if (scales.defined())
+  if (scales.defined()) {
+    const Recorded call("prefixlm::proj_gemm_scaled", {x, w, scales});
     check(lib.proj_gemm_scaled(&p, stream_of(x)), "prefixlm_proj_gemm_scaled");
-  else
+  } else {
+    const Recorded call("prefixlm::proj_gemm", {x, w});
     check(lib.proj_gemm(&p, stream_of(x)), "prefixlm_proj_gemm");
+  }
   return y;
 }
 // x, w, swiglu, norm, eps

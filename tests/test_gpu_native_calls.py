@@ -7,7 +7,7 @@ import torch
 from prefixlm import (_native, flash_attn_varlen_prefixlm, flash_attn_with_kvcache, fused_attention_layer, plan_inputs,
                       rms_norm, swiglu)
 from prefixlm.hrm_stack import rotary_cos_sin
-from prefixlm.norm_mlp import rms_norm_linear, rms_norm_swiglu
+from prefixlm.norm_mlp import add_rms_scales, rms_norm_linear, rms_norm_swiglu, rms_scaled_swiglu
 from prefixlm.synth import make_batch
 
 pytestmark = pytest.mark.gpu
@@ -226,3 +226,27 @@ def test_hooks_that_give_back_other_tensors(name, path):
         with pytest.raises(error):
             torch.autograd.grad(y, x, dy)
     assert given.count(True) == 1
+
+
+def test_the_profiler_sees_the_calls(path):
+    """torch.profiler shows each call and each backward under its operator's name, once, with shapes."""
+    b = make_batch([10, 30], [40, 20], 128, 2, 128, seed=5, device=DEV)
+    cos, sin = rotary_cos_sin(torch.arange(128, device=DEV), 128, 10000.0, 1024)
+    q, g = b.q.clone().requires_grad_(), _rand(128, 8, 128).requires_grad_()
+    x, gu, w = _rand(40, 256).requires_grad_(), _rand(40, 512, seed=1).requires_grad_(), _rand(512, 256, seed=2)
+    kq, cache = _rand(1, 1, 2, 128), _rand(2, 1, 64, 2, 128)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], record_shapes=True) as prof:
+        torch.autograd.grad(flash_attn_varlen_prefixlm(q, b.k, b.v, False, **b.seq_info), q, b.dout)
+        torch.autograd.grad(fused_attention_layer(g, cos, sin, False, **b.seq_info), g, b.dout)
+        torch.autograd.grad(rms_norm(x, 1e-6), x, _rand(40, 256, seed=3))
+        torch.autograd.grad(swiglu(gu), gu, _rand(40, 256, seed=3))
+        with torch.no_grad():
+            rms_norm_linear(x, w, 1e-6)
+            s, rstd = add_rms_scales(x, x, 1e-6)
+            rms_scaled_swiglu(s, w, rstd, 1e-6)
+            flash_attn_with_kvcache(kq, cache[0], cache[1], k=kq, v=kq, cache_seqlens=0)
+    seen = {e.key: e for e in prof.key_averages(group_by_input_shape=True) if e.key.startswith("prefixlm::")}
+    assert {k: e.count for k, e in seen.items()} == {f"prefixlm::{n}": 1 for n in (
+        "varlen_fwd", "varlen_bwd", "attn_layer_fwd", "attn_layer_bwd", "rms_norm_fwd", "rms_norm_bwd", "swiglu_fwd",
+        "swiglu_bwd", "proj_gemm", "add_rmsnorm", "proj_gemm_scaled", "kvcache_attn")}
+    assert seen["prefixlm::varlen_fwd"].input_shapes[0] == [128, 2, 128]
