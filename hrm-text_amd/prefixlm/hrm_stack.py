@@ -36,7 +36,7 @@ import torch
 import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 from torch import Tensor, nn
-from torch.nn.modules.module import _has_any_global_hook
+from torch.nn.modules import module as _nn_module
 
 __all__ = ["HRMStackConfig", "HRMStack", "FusedLayer", "rotary_cos_sin", "apply_rotary", "intermediate_size"]
 
@@ -192,8 +192,15 @@ class _Block(nn.Module):
 
 
 def _called_plainly(m: nn.Module, cls) -> bool:
-    return (type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks
-            and "forward" not in m.__dict__ and m._compiled_call_impl is None)
+    """Whether calling m runs cls.forward alone. What torch keeps its hooks in is private to it:
+    a version without these names counts as one with hooks."""
+    return (type(m) is cls and "forward" not in m.__dict__ and not getattr(m, "_forward_hooks", True)
+            and not getattr(m, "_forward_pre_hooks", True) and getattr(m, "_compiled_call_impl", m) is None)
+
+
+def _any_global_hook() -> bool:
+    has = getattr(_nn_module, "_has_any_global_hook", None)
+    return True if has is None else has()
 
 
 class _Module(nn.Module):
@@ -214,7 +221,7 @@ class _Module(nn.Module):
             if type(t) is not Tensor or t.device.type != "cuda" or t.dtype != torch.bfloat16 \
                     or fwAD.unpack_dual(t).tangent is not None:
                 return False
-        return (hidden.shape == injection.shape and hidden.device == injection.device and not _has_any_global_hook()
+        return (hidden.shape == injection.shape and hidden.device == injection.device and not _any_global_hook()
                 and all(_called_plainly(b, _Block) and _called_plainly(b.mlp, _SwiGLU) for b in self.layers))
 
     def _forward_fused_adds(self, hidden, injection, cos, sin, attn, seq_info):

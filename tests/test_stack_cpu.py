@@ -1,8 +1,12 @@
 """The HRM block stack around the op: structure and a tiny CPU run with a float32
 attention (no GPU)."""
+import importlib.util
+import sys
+
 import torch
 
 from oracle.prefixlm_oracle import attention_fwd
+from prefixlm import hrm_stack
 from prefixlm.hrm_stack import (HRMStack, HRMStackConfig, apply_rotary, intermediate_size,
                                 packed_position_ids, rotary_cos_sin)
 from prefixlm.synth import metadata_tensors
@@ -91,3 +95,23 @@ def test_only_the_window_records_gradients():
     y_all = model(x, pos, attn, {**st, **ss}, bp_steps=None)
     assert seen == [True] * 6
     torch.testing.assert_close(y_all, y)
+
+
+def test_imports_and_calls_blocks_without_torchs_private_names(monkeypatch):
+    """A torch that keeps its hooks elsewhere imports the stack, and its blocks count as hooked
+    (called one operation after another)."""
+    cfg = HRMStackConfig(hidden_size=64, num_heads=2, layers_per_module=1, max_seq_len=64)
+    assert not hrm_stack._any_global_hook()
+    monkeypatch.delattr(torch.nn.modules.module, "_has_any_global_hook")
+    spec = importlib.util.spec_from_file_location("prefixlm.stack_copy", hrm_stack.__file__)
+    copy = importlib.util.module_from_spec(spec)
+    monkeypatch.setitem(sys.modules, spec.name, copy)
+    spec.loader.exec_module(copy)
+    assert copy._any_global_hook()
+    block = copy._Block(cfg)
+    assert copy._called_plainly(block, copy._Block)
+    handle = block.register_forward_hook(lambda *a: None)
+    assert not copy._called_plainly(block, copy._Block)
+    handle.remove()
+    del block._forward_pre_hooks
+    assert not copy._called_plainly(block, copy._Block)
