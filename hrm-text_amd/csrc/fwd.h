@@ -82,7 +82,7 @@ struct Params {
   int n_main, total;
   // UNIFORM (a prefill of numseqs sequences of seq_len new rows each): no work list and no
   // metadata; the new rows of k and v also go to the caches
-  int seq_len;
+  int seq_len, seq_major;   // seq_major: the tiles of one sequence after another
   bf16* kc;
   bf16* vc;
   int64_t kc_sb, kc_ss, kc_sh, vc_sb, vc_ss, vc_sh;
@@ -186,12 +186,18 @@ __global__ __launch_bounds__(NT * KS, KS > 1 ? 2 : HD == 64 ? 4 : 3) void prefix
   }
   int item, h, seg, qt, cs, L, p;
   if constexpr (UNIFORM) {
-    // the last tiles first: with a causal mask they see the most keys
     const int tiles = (P.seq_len + BM - 1) / BM;
     if (!unit_of(blockIdx.x, P.numseqs * tiles, P.H, &item, &h)) return;
-    const int back = item / P.numseqs;
-    qt = tiles - 1 - back;
-    seg = item - back * P.numseqs;
+    if (P.seq_major) {
+      seg = item / tiles;
+      qt = item - seg * tiles;
+    } else {
+      // the last tiles of every sequence first: with a causal mask they see the most keys,
+      // without one they may be short and share a CU with a later one
+      const int back = item / P.numseqs;
+      qt = tiles - 1 - back;
+      seg = item - back * P.numseqs;
+    }
     cs = seg * P.seq_len;
     L = P.seq_len;
     p = P.is_causal ? 0 : L;

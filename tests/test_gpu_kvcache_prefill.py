@@ -27,3 +27,17 @@ def test_prefill_edges(B, S, H, Smax, causal):
     assert torch.equal(kd.cpu(), kr) and torch.equal(vd.cpu(), vr)
     err = (out.float().cpu() - ref).abs()
     assert (err <= ref.abs() * 2.0 ** -8 + v.abs().max().item() * 2.0 ** -9).all(), f"max_abs {err.max().item():.3e}"
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_prefill_of_more_tiles_than_the_chip_holds(causal):
+    """17 sequences x 3 tiles x 20 heads: one sequence after another without a causal mask."""
+    B, S, H = 17, 300, 20
+    g = torch.Generator().manual_seed(S)
+    q, k, v, kc, vc = (torch.randn(B, S, H, 128, generator=g).to(torch.bfloat16) for _ in range(5))
+    ref, kr, vr = kvcache_attention(q, kc, vc, k, v, 0, causal)
+    kd, vd = kc.to(DEV), vc.to(DEV)
+    out = flash_attn_with_kvcache(q.to(DEV), kd, vd, k=k.to(DEV), v=v.to(DEV), cache_seqlens=0, causal=causal)
+    assert torch.equal(kd.cpu(), kr) and torch.equal(vd.cpu(), vr)
+    err = (out.float().cpu() - ref).abs()
+    assert (err <= ref.abs() * 2.0 ** -8 + v.abs().max().item() * 2.0 ** -9).all(), f"max_abs {err.max().item():.3e}"
