@@ -51,12 +51,14 @@ __device__ __forceinline__ void store_row(bf16* p, bf16x8 v) {
   else
     *q = __builtin_bit_cast(u32x4, v);
 }
-// Inputs and outputs above the 256 MB of the last-level cache: nothing of them was left
-// there by their producer or can be left for their reader, so the kernels neither look nor
-// allocate there. Below it the plain forms are as fast or faster (4096 x 3584 columns
-// forward 14.1 us plain, 15.9 non-temporal); above it: 16384 x 5632 forward 93 -> 86 us (6.4
-// TB/s), backward 161 -> 143 us (6.4 TB/s); 51620 x 7784 420 -> 383 and 768 -> 715 us.
-constexpr int64_t kNtBytes = (int64_t)256 << 20;
+// Inputs and outputs above what the caches hold (256 MB in the last level, 32 MB in the L2s):
+// nothing of them was left there by their producer or can be left for their reader, so the
+// kernels neither look nor allocate there. Below it the plain forms are as fast or faster
+// (forward 8192 x 5632 columns, 264 MB, 39.8 us plain and 42.7 non-temporal; backward 7000 x
+// 4096, 273 MB, 42.4 and 45.0); above it: forward 12288 x 4096, 288 MB, 50.0 and 46.2, 16384 x
+// 5632 93 and 84.6 (6.5 TB/s); backward 8192 x 4096, 320 MB, 58.7 and 53.1, 16384 x 5632 161 and
+// 142 (6.5 TB/s). Between the products of an MLP either form takes the same within 2%.
+constexpr int64_t kNtBytes = (int64_t)280 << 20;
 
 // thread = 8 consecutive columns of one row
 template <bool NT>
