@@ -1,5 +1,5 @@
 """GPU: KV-cache attention at both sides of the lines where a call gives up splitting the keys
-(decode: caches of 384 rows, 128 (row, head) pairs; several new rows: the tiles against the
+(decode: caches of 384 and 1088 rows, 128 (row, head) pairs; several new rows: the tiles against the
 partials) or change a decode workgroup's size (64 cache rows, 256 pairs), with empty, ragged and full caches, against the oracle.
 
 Tolerance per element: half a bf16 ulp of the reference (2^-8 |ref|, the output's own rounding)
@@ -17,6 +17,7 @@ DEV = torch.device("cuda:0")
 @pytest.mark.parametrize("B,S,H,Smax", [
     (1, 1, 1, 1), (2, 1, 3, 64), (2, 1, 3, 65), (3, 1, 3, 127), (3, 1, 3, 129), (2, 1, 3, 384), (2, 1, 3, 385),
     (8, 1, 16, 384), (129, 1, 1, 384), (256, 1, 1, 300), (257, 1, 1, 300), (16, 1, 16, 1023),
+    (9, 1, 16, 1087), (9, 1, 16, 1088), (18, 1, 20, 1090),
     (1, 5, 8, 128), (1, 5, 8, 256), (1, 5, 8, 257), (1, 64, 8, 128), (1, 64, 8, 129), (4, 64, 16, 512),
     (4, 64, 16, 513), (4, 100, 16, 256), (4, 100, 16, 480), (16, 33, 16, 200), (16, 20, 8, 500)])
 def test_matches_oracle(B, S, H, Smax):
