@@ -41,7 +41,7 @@ def _run(q, k, v, kc, vc, lens, causal):
 @pytest.mark.parametrize("S", [1, 3])
 @pytest.mark.parametrize("causal", [False, True])
 def test_decode_matches_oracle(S, causal):
-    B, H, Smax = 5, 4, 1100          # three 512-key splits, the last one partial
+    B, H, Smax = 5, 4, 1100          # 18 splits of one 64-key step, or 9 of one 128-key tile
     print(f"[kvcache] decode S={S} causal={causal}", flush=True)
     q, k, v, kc, vc = _inputs(B, S, H, Smax, 10 + S)
     lens = torch.tensor([0, 1, 511, 900, Smax - S], dtype=torch.int32)

@@ -32,7 +32,8 @@ def _run(B, H, Smax, lens, shared=False):
     assert (err <= tol).all(), f"max_abs {err.max().item():.3e}"
 
 
-# 12 splits; 64 splits of one step; one split of a short cache in a batch that fills the chip
+# 11 splits of one step; 64 splits of 128 keys, the last 24 without keys; one split of a short cache in
+# a batch that fills the chip
 @pytest.mark.parametrize("B,H,Smax", [(9, 5, 700), (1, 2, 5000), (130, 2, 129)])
 def test_decode_lengths(B, H, Smax):
     edges = [0, 1, 63, 64, 65, 127, 128, Smax // 2, Smax - 1, Smax]

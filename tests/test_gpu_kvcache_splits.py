@@ -3,7 +3,7 @@
 partials) or change a decode workgroup's size (64 cache rows, 256 pairs), with empty, ragged and full caches, against the oracle.
 
 Tolerance per element: half a bf16 ulp of the reference (2^-8 |ref|, the output's own rounding)
-plus 2^-14 max|V| for fp32 sums in another order and probabilities carried to 16 bits."""
+plus 2^-14 max|V| for fp32 sums in another order."""
 import pytest
 import torch
 

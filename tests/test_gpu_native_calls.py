@@ -1,6 +1,7 @@
 """GPU: the native host path of the public calls against the Python path they replace:
 bitwise the same results and gradients, the same refusals, and the calls it hands back
-(operands that need a copy, recorded and batched backwards, modes, saved-tensor hooks)."""
+(operands that need a copy, recorded and batched backwards, dispatch and function modes,
+saved-tensor hooks that give back other tensors)."""
 import pytest
 import torch
 
@@ -250,3 +251,74 @@ def test_the_profiler_sees_the_calls(path):
         "varlen_fwd", "varlen_bwd", "attn_layer_fwd", "attn_layer_bwd", "rms_norm_fwd", "rms_norm_bwd", "swiglu_fwd",
         "swiglu_bwd", "proj_gemm", "add_rmsnorm", "proj_gemm_scaled", "kvcache_attn")}
     assert seen["prefixlm::varlen_fwd"].input_shapes[0] == [128, 2, 128]
+
+
+def _call(name, plan):
+    """(leaf input, call, output gradient) of one differentiable call."""
+    T, H = 300, 2
+    b = make_batch([60, 20], [100, 70], T, H, 128, seed=6, device=DEV)
+    info = {**b.seq_info, **(plan_inputs(b.seq_tensors, b.seq_scalars, DEV) if plan else {})}
+    cos, sin = rotary_cos_sin(torch.arange(T, device=DEV), 128, 10000.0, 1024)
+    x, f, dy = {
+        "varlen": (b.q, lambda q: flash_attn_varlen_prefixlm(q, b.k, b.v, False, **info), b.dout),
+        "layer": (_rand(T, 4 * H, 128, seed=1), lambda g: fused_attention_layer(g, cos, sin, False, **info), b.dout),
+        "rms_norm": (_rand(40, 256, seed=1), lambda x: rms_norm(x, 1e-6), _rand(40, 256, seed=2)),
+        "swiglu": (_rand(40, 512, seed=1), swiglu, _rand(40, 256, seed=2)),
+    }[name]
+    return x.clone().requires_grad_(), f, dy
+
+
+CALLS = [("varlen", False), ("varlen", True), ("layer", False), ("layer", True), ("rms_norm", False), ("swiglu", False)]
+
+
+@pytest.mark.parametrize("name,plan", CALLS)
+def test_recorded_backwards_give_the_same_gradient(name, plan):
+    """create_graph takes the custom op, whose arguments the native node lines up by hand."""
+    assert _native.calls() is not None
+    x, f, dy = _call(name, plan)
+    want, = torch.autograd.grad(f(x), x, dy)
+    got, = torch.autograd.grad(f(x), x, dy.clone().requires_grad_(), create_graph=True)
+    assert got.requires_grad and torch.equal(got.detach(), want)
+
+
+@pytest.mark.parametrize("name,plan", CALLS)
+def test_modes_see_the_operators(name, plan):
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    assert _native.calls() is not None
+    seen = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x, f, dy = _call(name, plan)
+    y = f(x)
+    want, = torch.autograd.grad(y, x, dy)
+    for mode in (Dispatch, Function):
+        with mode():
+            z = f(x)
+            got, = torch.autograd.grad(z, x, dy)
+        assert torch.equal(z, y) and torch.equal(got, want)
+    assert sum(op.startswith("prefixlm.") for op in seen) == 2
+
+
+@pytest.mark.parametrize("name,plan", CALLS)
+def test_batched_gradients_as_on_the_python_path(name, plan, monkeypatch):
+    def run():
+        x, f, dy = _call(name, plan)
+        try:
+            return torch.autograd.grad(f(x), x, torch.stack((dy, 2 * dy)), is_grads_batched=True)[0]
+        except Exception as e:
+            return type(e)
+    assert _native.calls() is not None
+    a = run()
+    with monkeypatch.context() as m:
+        m.setattr(_native, "_module", None)
+        b = run()
+    assert torch.equal(a, b) if isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor) else a is b
