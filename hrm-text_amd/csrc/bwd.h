@@ -1125,7 +1125,7 @@ __global__ __launch_bounds__(q2::NT, 3) void prefixlm_bwd_dq_ds_kernel(Q2Params 
 // =====================================================================================
 // pre-pass and padding rows
 // =====================================================================================
-constexpr int kPreRows = 32;     // token rows per pre-pass workgroup, at most (see pre_rows)
+constexpr int kPreRows = 32;     // token rows per pre-pass workgroup, at most (fewer where that leaves CUs idle: see the launch)
 constexpr int kPreBatch = 8;     // row-heads per 16-lane group whose loads are in flight together
 constexpr int kPreMaxHeads = 64; // per-head maxima kept in LDS
 

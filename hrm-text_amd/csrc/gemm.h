@@ -26,9 +26,10 @@
 //
 // Bound by the board's power at large M (a stage takes the same 2700 cycles at any load, at
 // 2.4 GHz for 44 workgroups and about 1.75 with every CU busy), by the fill of the CUs at small
-// M. K 2048, N 11264 with SwiGLU: M 16384 642 us (1.18 PFLOP/s), M 1100 51 us. Before (a
-// workgroup per tile, m tiles dealt to the XCDs by number, a stage's direct loads issued in
-// one burst): 656 and 102 us: five m tiles kept three XCDs idle and gave the others two rounds.
+// M. K 2048, N 11264 with SwiGLU, the norm's pass included: M 16384 615 us (1.23 PFLOP/s; 609 to
+// 634 on different cards), M 1100 55 us. A workgroup per tile, m tiles dealt to the XCDs by number
+// and a stage's direct loads issued in one burst took 2% more and twice as long: five m tiles kept
+// three XCDs idle and gave the others two rounds.
 #pragma once
 #include "common.h"
 
@@ -292,9 +293,9 @@ __global__ __launch_bounds__(NTH, 1) void proj_gemm_kernel(Params P) {
 // of every tile. The row scales come from the x fragments on the way, so the norm needs no
 // launch of its own.
 // Bound by the stream of W up to 32 rows, by the repeated reads of x from L2 above: K 2048,
-// N 11264 (46 MB) 11.5 us for 1 row and 12.8 for 16 (4 TB/s), 18.7 for 64, 24.5 for 100; the
-// 128-row tiles take 32 us for any of them (44 workgroups), which x reads would reach past
-// 128 rows.
+// N 11264 (46 MB) with SwiGLU 11.6 us for 1 row and 12.7 for 16 (3.7 TB/s), 18.9 for 64, 29.0 for
+// 100 and 29.3 for 128; the 128-row tiles take 36 us for any of them (44 workgroups), which x reads
+// would reach past 128 rows.
 template <int MB, int NWV>
 struct SkinnyGeo {
   static constexpr int TILE = 64 * 16 * 4;       // one wave's partial 32 x 32 tile

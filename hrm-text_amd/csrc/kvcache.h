@@ -91,8 +91,10 @@ __device__ __forceinline__ u32x4 load_once(const bf16* p) {
 }
 
 // One query per row (S = 1): blockIdx.x = ((b * H + h) * nsplit + split). The splits share
-// each sequence's own length evenly (in steps of 64 keys), so a ragged batch has no
-// workgroups without keys beside full ones. Bound by HBM. The cache loads are non-temporal:
+// each sequence's own length, in whole steps of 64 keys: all but the last with keys hold the
+// same number, and those past the length none (4200 keys in 64 splits: 128 each in 33 of them). A
+// ragged batch so has no sequence whose splits are all full beside one whose splits are mostly
+// empty, as splits of fixed 512 keys had. Bound by HBM. The cache loads are non-temporal:
 // a row is read once, and kept out of the caches it costs no write-back of what it would
 // evict. 64 x 16 heads, 2100-4000 of 4096 rows (1.6 GB): 262 us with the combine, 6.1 TB/s,
 // against 285 with plain loads and 322 for fixed 512-key splits, plain loads and an append
@@ -251,8 +253,9 @@ __global__ __launch_bounds__(NTH) void decode_kernel(Params P) {
 // Bound by HBM (512 bytes per key and query block) up to about 64 queries, by the MFMA ->
 // softmax -> MFMA chain above. Measured against the walk of the queries one after another that
 // this replaces (each query read all keys again): 4 x 16 heads x 45 queries on 4096-row half
-// full caches 658 -> 24 us; 16 x 16 x 512 queries on 8192-row caches 0.70 ms (466 TFLOP/s
-// useful). Two workgroups per CU: at three (168 VGPRs) the 128-query form spills, 0.85 ms.
+// full caches 658 -> 28 us with the combine; 16 x 16 x 512 queries on 7000 of 8192 rows 1.11 ms (437
+// TFLOP/s useful). Two workgroups per CU: at three (168 VGPRs) the 128-query form spills, a fifth
+// slower.
 //
 // New rows (keys len .. len + S - 1) are read from k, v, and every workgroup copies its
 // share of them into the caches: nothing in the launch reads those cache rows, so no

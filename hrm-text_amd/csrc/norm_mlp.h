@@ -130,8 +130,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 // one wave per row, 4 rows per workgroup; the row stays in registers between the passes
 // (NCH 16-byte chunks per lane, the smallest power of two covering the row). ADD: the block's
 // residual add in the same pass, so that s is not read back and one launch is left of two; bound
-// by memory. 1100 rows of 2048: 6.3 us (5.5 without y) against 9.5 for the add and the norm apart,
-// 16384 rows 43 (34; 6.2 TB/s) against 54.
+// by memory. 1100 rows of 2048: 4.7 us (3.9 without y) against 8.4 for the add and the norm apart,
+// 16384 rows 41 (31; 6.5 TB/s) against 50.
 template <int NCH, bool ADD = false>
 __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(NormParams P) {
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);

@@ -1018,9 +1018,9 @@ static int proj_gemm_launch(const prefixlm_proj_gemm_args* a, void* stream_, boo
                 a->rstd, a->x_stride, a->w_stride, a->y_stride, a->M, a->K, a->N, 0, 0};
   P.n_tiles = a->N / mlp::WT;
   // 256 x rows per tile, or 128 where that needs fewer or shorter rounds over the CUs: a round
-  // of 128-row tiles takes 0.65 (many rounds) to 0.8 (one) of a round of 256-row ones, the W
-  // tile's loads staying the same (K 2048, N 11264: M 512 34 us with 128 rows, 44 with 256;
-  // M 700 65 and 45; M 1100 70 and 51; M 16384 832 and 642)
+  // of 128-row tiles takes 0.6 (many rounds) to 0.8 (one) of a round of 256-row ones, the W
+  // tile's loads staying the same (K 2048, N 11264: M 512 37 us with 128 rows, 47 with 256;
+  // M 700 67 and 49; M 1100 74 and 54; M 16384 748 and 614)
   const int64_t t256 = (int64_t)((a->M + 255) / 256) * P.n_tiles, t128 = (int64_t)((a->M + 127) / 128) * P.n_tiles;
   if (t128 > 0x7fffffff) return fail(PREFIXLM_ERR_INVALID, "grid too large");
   const bool half = 7 * ((t128 + cus - 1) / cus) < 10 * ((t256 + cus - 1) / cus);
@@ -1098,17 +1098,19 @@ static int64_t kv_nsplit(int64_t B, int S, int64_t H, int64_t Smax) {
     return std::max<int64_t>(1, std::min(std::max<int64_t>(2, (1024 + units - 1) / units), most));
   }
   const int64_t tk = 32 * (4 / ext_qw(S)), units = B * H * kv_nqb(S);
-  // 512 workgroups fill the chip (two per CU); more splits only add partials to write and
-  // merge: 4 x 16 heads x 45 queries 38 us a call at 512, 42 at 1024, 60 at 2048, and 2 x 16 x
-  // 300 on 8192 rows 97 us at 512 against 103 at 256
+  // 512 workgroups fill the chip (two per CU); more splits mostly add partials to write and
+  // merge: 4 x 16 heads x 45 queries 31 us at 512, 41 at 1024, 58 at 2048, and 2 x 16 x 300 on
+  // 8192 rows 119 us at 256, 103 at 512, 97 at 1024, 115 at 2048
   const int64_t want = (512 + units - 1) / units, most = (Smax + tk - 1) / tk;
   const int64_t n = std::max<int64_t>(1, std::min({want, most, (int64_t)kvc::kMaxSplits}));
   // One split instead where the tiles it walks more cost less than the combine's launch and the
-  // partials, which n splits write and read for every query. Measured: a tile of 32, 64 or 128
+  // partials, which n splits write and read for every query. The estimate: a tile of 32, 64 or 128
   // keys takes 1.27, 1.5 or 2.1 us with up to 512 workgroups, the launch 2.1 us at the least,
-  // a partial 0.2 ns. 256 pairs x 64 queries, one split against two: 128-row caches 15.4 and
-  // 32.0 us, 512 28.7 and 39.8, 1024 39.6 and 46.7; 64 pairs x 128 queries on 256 rows 24.1, and
-  // 28.3 with eight; 8 pairs x 64 queries on 256 rows 16.5, and 12.9 with the four it keeps.
+  // a partial 0.2 ns. 256 pairs x 64 queries, one split against two: 128-row caches 15.0 and
+  // 32.6 us, 512 29.3 and 41.5; 64 pairs x 128 queries on 256 rows 24.9, and 29.8 with eight; 8
+  // pairs x 64 queries on 256 rows 16.4, and 13.8 with the four it keeps. It errs beside its line
+  // (256 pairs x 64 queries on 1024 rows 53.5 with the two it keeps, 44.0 with one), but 0.35 ns a
+  // partial, right there, makes others worse (12 pairs x 200 queries on 200 rows 17.1 -> 22.1).
   const double c = ext_qw(S) == 1 ? 2100 : ext_qw(S) == 2 ? 1500 : 1270;   // ns
   const double one = (double)most * c * std::max(1.0, (double)units / 512);
   const double split = (double)((most + n - 1) / n) * c * std::max(1.0, (double)units * (double)n / 512) + 2100 +

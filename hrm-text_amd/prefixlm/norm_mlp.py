@@ -275,9 +275,10 @@ def _proj(x: Tensor, w: Tensor, swiglu: bool, eps: float) -> Tensor:
 def rms_norm_linear(x: Tensor, w: Tensor, eps: float) -> Tensor:
     """F.linear(F.rms_norm(x, (K,), eps), w) in one GEMM (forward only).
 
-    Faster than the norm kernel plus the library's GEMM for few rows, slower for many: at
-    2048 -> 8192 columns 8.9 against 24.3 us for 16 rows, 23.1 and 24.9 for 128, 33.8 and
-    26.4 for 512, 493 and 414 for 16384. The normalized activations are never written."""
+    Against the norm kernel plus the library's GEMM, both queued, at 2048 -> 8192 columns: 9.0
+    and 12.1 us for 16 rows, 15.0 and 14.1 for 64, 23.8 and 17.4 for 128, 35.6 and 27.0 for 512,
+    477 and 412 for 16384. The normalized activations are never written, and one call costs the
+    host less than two."""
     return _proj(x, w, False, float(eps))
 
 
@@ -285,10 +286,10 @@ def rms_norm_swiglu(x: Tensor, w_gate_up: Tensor, eps: float) -> Tensor:
     """silu(g) * u for [g | u] = F.linear(F.rms_norm(x, (K,), eps), w_gate_up), in one
     GEMM (forward only).
 
-    Against the norm kernel, the library's GEMM and the SwiGLU kernel, at 2048 -> 11264
-    columns: 12.4 and 29.2 us for 16 rows, 54 and 58 for 1100, 162 and 188 for 4096, 617
-    and 645 for 16384 (the GEMM core is slower than the library's, 1.2 against 1.4 PFLOP/s,
-    and the two elementwise passes make up for it)."""
+    Against the norm kernel, the library's GEMM and the SwiGLU kernel, all queued, at 2048 ->
+    11264 columns: 12.7 and 15.9 us for 16 rows, 29.3 and 22.0 for 128, 38 and 39 for 512, 55 and
+    60 for 1100, 164 and 191 for 4096, 612 and 639 for 16384 (the GEMM core is slower than the
+    library's, 1.2 against 1.4 PFLOP/s, and the two elementwise passes make up for it)."""
     return _proj(x, w_gate_up, True, float(eps))
 
 
